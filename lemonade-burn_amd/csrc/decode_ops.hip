@@ -988,15 +988,22 @@ int launch_attention(lbt_ctx* ctx, const float* q, int m, int nh, int kvh, int h
                      const uint16_t* kc, const uint16_t* vc, int cap, float scaling, float* o, float* ml,
                      bool grouped) {
     if (kvh <= 0 || nh % kvh) return set_err(ctx, LBT_E_INVALID, "attention: heads must be a multiple of kv heads");
+    // a prefill's rows in 16-row tiles on the matrix cores, where that is the
+    // faster (its rule); LBT_ATTN_TILE=1 / 0 forces it on / off
+    if (ctx->tune.attn_tile > 0 || (ctx->tune.attn_tile < 0 && ctx->tune.attn_wave < 0)) {
+        const int rc = launch_attention_tile(ctx, q, m, nh, kvh, hd, rp, kc, vc, cap, scaling, o, ml);
+        if (rc != 1) return rc;
+    }
     const int gh = nh / kvh;
     if (gh != 1 && gh != 2 && gh != 4) grouped = false;
     const size_t lds = grouped ? (size_t)gh * attn_group_score_keys(attn_split_keys(rp.vis_max), hd / 8) * sizeof(float)
                                : (size_t)attn_split_keys(rp.vis_max) * sizeof(float);
     if (lds > 64 * 1024) return set_err(ctx, LBT_E_RANGE, "attention: context too long for the LDS score buffer");
     // rows of one sequence at consecutive positions (a prefill) with at
-    // least 8 (row, KV head, split) tasks per CU: one wavefront per task
-    // where the shape allows (2B, 2048-token prefill: attention 41.5 ->
-    // 18.9 ms; at 64 and 128 tokens the workgroup per task stays faster,
+    // least 8 (row, KV head, split) tasks per CU that the tile kernel does not
+    // take (splits of more than 256 keys, contexts past 4096): one wavefront
+    // per task where the shape allows (2B, 2048-token prefill: attention 41.5
+    // -> 18.9 ms; at 64 and 128 tokens the workgroup per task stays faster,
     // 0.25 against 0.42 ms and 0.38 against 0.43 ms).  LBT_ATTN_WAVE=1 / 0
     // forces it on / off for grouped attention.
     const int aw = ctx->tune.attn_wave;

@@ -34,6 +34,10 @@ LbtTuning read_tuning() {
         t.attn_wave = v ? (atoi(v) != 0 ? 1 : 0) : -1;
     }
     {
+        const char* v = getenv("LBT_ATTN_TILE");
+        t.attn_tile = v ? (atoi(v) != 0 ? 1 : 0) : -1;
+    }
+    {
         const char* v = getenv("LBT_ATTN_WIDE");
         t.attn_wide = v ? (atoi(v) != 0 ? 1 : 0) : -1;
     }

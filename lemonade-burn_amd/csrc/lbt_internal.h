@@ -24,6 +24,7 @@ struct LbtTuning {
     int small_ns = 0;         // LBT_GEMM_SMALL_NS: 1 / 2 forces its row tile (0 auto)
     bool small_pf = true;     // LBT_GEMM_SMALL_PF=0: no epilogue prefetch
     int attn_wave = -1;       // LBT_ATTN_WAVE=1/0: one wavefront per (row, KV head, split) on/off (-1: prefill rows)
+    int attn_tile = -1;       // LBT_ATTN_TILE=1/0: 16-row attention tiles on the matrix cores on/off (-1: by grid size)
     int attn_wide = -1;       // LBT_ATTN_WIDE=1/0: eight-pass K/V pipeline of the grouped attention on/off (-1: by grid size)
     bool head_tg8 = false;           // LBT_HEAD_TG8: 8-token groups in the batched LM head
     bool head_batch_classic = false;  // LBT_HEAD_BATCH_CLASSIC: batched bf16 head on lmhead_batch_kernel (16-token groups)
@@ -249,6 +250,11 @@ __host__ __device__ __forceinline__ size_t row_cache_offset(const RowPos& r, int
 int launch_attention(lbt_ctx* ctx, const float* q, int m, int nh, int kvh, int hd, const RowPos& rp,
                      const uint16_t* kc, const uint16_t* vc, int cap, float scaling, float* o, float* ml,
                      bool grouped = false);
+// The same splits of a prefill's rows (consecutive positions of one sequence,
+// head_dim 128, splits of up to 256 keys) on the f32 matrix cores, the same
+// bits; returns 1 (nothing launched) for what it does not take.
+int launch_attention_tile(lbt_ctx* ctx, const float* q, int m, int nh, int kvh, int hd, const RowPos& rp,
+                          const uint16_t* kc, const uint16_t* vc, int cap, float scaling, float* o, float* ml);
 // Combine of the splits into out [m][nh*hd].
 int launch_attn_combine(lbt_ctx* ctx, const float* o, const float* ml, int m, int nh, int hd, const RowPos& rp,
                         float* out);
