@@ -1300,8 +1300,7 @@ int launch_ternary_mfma(lbt_ctx* ctx, const TernaryOp& op_in) {
     // few-token kernel, 4 / 5 = 64 / 128 tiles of the pipelined GEMM, 7 / 8 =
     // the 128 x 256 / 64 x 320 tiles of one workgroup per CU; by default the
     // few-token kernel up to tune.small_max tokens, then the one-workgroup-
-    // per-CU tiles as picked below, else 128 x 128 tiles when there are
-    // >= 200, else 64 x 64
+    // per-CU tiles as picked below, else 128 x 128 or 64 x 64 tiles
     const LbtTuning& tu = ctx->tune;
     const int gmode = tu.gemm_mode;
     const long t128 = (long)((total + 127) / 128) * ((op.m + 127) / 128);
@@ -1319,14 +1318,23 @@ int launch_ternary_mfma(lbt_ctx* ctx, const TernaryOp& op_in) {
     // of 2 x 2 per SIMD, two workgroups per CU), 1 per 64 x 64 tile; ties go
     // to the one-workgroup-per-CU kernel
     const long c3 = (t3 + 255) / 256 * 8, c3n = (t3n + 255) / 256 * 6;
-    const long c2 = t128 >= 200 ? (t128 + 255) / 256 * 4 : ((long)g64.x * g64.y + 255) / 256;
+    // 128 x 128 or 64 x 64 tiles: a round of 64 x 64 costs 1.6 (half the reuse
+    // of either operand), and 128 x 128 tiles that leave each CU at most one
+    // workgroup, one wavefront per SIMD, 4.6 instead of 4, 5.6 with the q/k/v
+    // epilogue (2B shape, o and down at 850 tokens, 140 tiles: 22.5 us against 26.6
+    // on 560 of 64 x 64; at 768, 480 of them in two rounds: 22.4 against 18.7;
+    // q/k/v at 768: 27.5 against 25.1, at 850: 27.8 against 29.6)
+    const long t64 = (long)g64.x * g64.y;
+    const long c64 = (t64 + 255) / 256 * 16;
+    const long c128 = t128 > 256 ? (t128 + 255) / 256 * 40 : op.out_mode == kOutQKV ? 56 : 46;
+    const bool use128 = c128 <= c64;
+    const long c2 = use128 ? (t128 + 255) / 256 * 4 : (t64 + 255) / 256;
     int g3pick = c3n < c3 ? (t3n >= kG3MinTiles ? 2 : 0) : (t3 >= kG3MinTiles ? 1 : 0);
     if (g3pick != 0 && (g3pick == 2 ? c3n : c3) > c2) g3pick = 0;
     const bool small_ok = a.kp <= 256 * 4 * kSmallMaxSteps;
     // up to 64 tokens the few-token kernel also serves the shapes the 64 x 64
     // tiling would give fewer than tune.small_tiles tiles (q/k/v, o, down of
     // the 2B model at B = 33..64)
-    const long t64 = (long)((total + 63) / 64) * ((op.m + 63) / 64);
     const bool few_tiles = op.m <= 64 && t64 < tu.small_tiles;
     if (small_ok && (gmode == 6 || (gmode == 0 && (op.m <= tu.small_max || few_tiles)))) {
         // 16-token tiles (more workgroups) measured faster than 32..64-token
@@ -1359,7 +1367,7 @@ int launch_ternary_mfma(lbt_ctx* ctx, const TernaryOp& op_in) {
             e = launch_tiles3<1, 10, 2, 1, 1, kG3Stages>(a, op.out_mode, g3n, ctx->stream, e0, e1);
         else
             e = launch_tiles3<1, 8, 4, 1, 1, kG3Stages>(a, op.out_mode, g3, ctx->stream, e0, e1);
-    } else if (gmode != 4 && (t128 >= 200 || gmode == 5)) {
+    } else if (gmode != 4 && (use128 || gmode == 5)) {
         // grids that leave workgroup slots idle split k (gridDim.z ranges)
         dim3 g = g128;
         pick_ksplit(ctx, op, a, t128, 4 * 4 * 1024, a.kp / 128);
@@ -1367,7 +1375,7 @@ int launch_ternary_mfma(lbt_ctx* ctx, const TernaryOp& op_in) {
         e = launch_tiles2<2, 2, 1>(a, op.out_mode, g, ctx->stream, e0, e1);
     } else {
         dim3 g = g64;
-        pick_ksplit(ctx, op, a, (long)g64.x * g64.y, 4 * 1024, a.kp / 128);
+        pick_ksplit(ctx, op, a, t64, 4 * 1024, a.kp / 128);
         g.z = (unsigned)a.ksplit;
         e = launch_tiles2<1, 1, 1>(a, op.out_mode, g, ctx->stream, e0, e1);
     }
