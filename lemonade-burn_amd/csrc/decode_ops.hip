@@ -942,7 +942,7 @@ int launch_head(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int 
         }
     }
     if (m >= 2 && (xn || !norm_w) && cols <= 64 * kLmChunks * 8 && ((uintptr_t)x & 15) == 0) {
-        // few rows of few or ragged columns (launch_head_tile's rule), and the switches;
+        // small matrices (launch_head_tile's rule), and the switches;
         // more than 8 rows: 16-token groups on 512 threads (the whole LDS of a
         // CU; each weight row is then read from L2 half as often), else
         // 8-token groups on 256 threads (two workgroups per CU)

@@ -7,260 +7,254 @@
 // The one-token head gives lane l of a wavefront the row's 8-element chunks
 // l, l + 64, ...: a chain of fused multiply-adds in element order, then the
 // 64 chains combine by an xor butterfly over 32, 16, 8, 4, 2, 1.
-// v_mfma_f32_16x16x1_4b does one fused multiply-add of four such chains for
-// 16 token rows x 16 weight rows (block b of an accumulator is one chain;
-// each step correctly rounded, checked on this part against fmaf), so a
-// chain of them is the lane's chain.  With l = 8 q + 2 b + a, accumulator
-// (q, a) holds the chains of blocks b = 0..3; the butterfly's pairs are then
-// q ^ 4, q ^ 2, q ^ 1 (whole accumulators), b ^ 2, b ^ 1 (blocks) and a.
+// v_mfma_f32_4x4x1_16b does one fused multiply-add of sixteen such chains for
+// 4 token rows x 4 weight rows (block k of an accumulator is one chain; each
+// step correctly rounded, denormals kept, checked on this part against fmaf),
+// so a chain of them is the lane's chain.  With l = 16 g + k, accumulator g
+// holds the chains of blocks k = 0..15; the butterfly's pairs are then g ^ 2,
+// g ^ 1 (accumulators) and lanes 32, 16, 8, 4 apart (lane 4 k + j), by
+// recursive halving of a wavefront's sums.
 #include <hip/hip_runtime.h>
 
 #include "lbt_device.h"
 #include "lbt_internal.h"
 
+#include <type_traits>
+
 namespace lbt {
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kTok = 16;       // token rows per workgroup
-constexpr int kVoc = 16;       // weight rows per wavefront and tile
-constexpr int kNT = 512;       // two wavefronts per SIMD, wavefront q the chains 8 q ..
-constexpr int kMaxNch = 5;     // chunks per chain (columns up to 2560: 80 registers of a token row)
-
-__device__ __forceinline__ f32x16 outer4(float a, float b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
-}
+constexpr int kMaxNch = 5;  // chunks per chain: columns up to 2560 (16 rows of f32 fill the LDS)
 
 }  // namespace
 
-// Eight wavefronts, one tile of 16 weight rows at a time for 16 token rows:
-// wavefront q has the chains 8 q .. 8 q + 7.  Its part of the token rows
-// (80 registers at 2560 columns) stays in registers, so the matrix
-// instructions take both operands from there; of each weight row it reads
-// 128 contiguous bytes (bf16) out of every 1024, and the eight wavefronts
-// together whole rows.  Weight chunks are reloaded for the tile after the
-// next as soon as they are used (20 KB in flight a wavefront, 160 KB a CU).
-// The accumulators meet in LDS (64 KB a tile, two tiles' worth, one barrier
-// a tile); a lane then adds one (token, row) sum's chains of one a.
-// Workgroup i takes token group i / ntw of row part i % ntw: with ntw a
-// multiple of 8 the groups of a part run on one XCD and share its L2's copy
-// of the weights.
+// 4 TG token rows in LDS (16-byte granule x of row t at x ^ ((t & 1) + 4 (t &
+// 2)), so four rows' reads of four chunks fall on distinct banks), a
+// wavefront takes tiles of 4 RG weight rows: a load is 256 contiguous bytes
+// (bf16) of each of 4 rows, RING steps ahead of the matrix instructions (64 to
+// 160 KB in flight a CU).  Up to 8 rows two workgroups of four wavefronts a
+// CU, above one of eight (16 rows fill its LDS; RG = 2 there and RING = 2 at
+// 12 rows of bf16 keep the sums in registers).  Workgroup i takes token group i / ntw of row part i % ntw: with
+// ntw a multiple of 8 the groups of a part run on one XCD and share its L2's
+// copy of the weights.
 //
-// Bound by the f32 multiply-adds (68 us per 16 rows and 128256 x 2560, used or
-// not) with the widening after them (the two take turns on a SIMD), and up to
-// 16 rows of bf16 by HBM beside them (657 MB, 100 us).  128256 x 2560: 16
-// rows 210 -> 160 us (lmhead_batch_kernel with the next weights in flight ->
-// this), 24 rows 360 -> 256, 64 rows 700 -> 460; int8 weights 16 rows 190 ->
-// 135, 64 rows 710 -> 494.  Measured beside it: the token rows in LDS and a
-// whole 16 x 16 tile a wavefront (16 rows 160, 64 rows 555; with 64-byte
-// pieces of a row a load 200), and the exchange's reads and barrier right
-// after its writes (64 rows 520).
-template <int NCH, bool FULL, bool Q8>
-__global__ __launch_bounds__(kNT) void lmhead_tile_kernel(const void* W, const float* rscale, int rows, int cols,
-                                                          const float* xn, int m, int part_tiles, float* logits,
-                                                          unsigned long long* key) {
-    constexpr int NV = Q8 ? 1 : 2;  // 16-byte loads of a lane's two chunks
-    extern __shared__ __align__(16) float part_s[];  // [2][q][a][16 registers][64 lanes]
-    const int ngroups = (m + kTok - 1) / kTok, ntw = (int)gridDim.x / ngroups;
-    const int grp = (int)blockIdx.x / ntw, part = (int)blockIdx.x % ntw;
-    const int t0 = grp * kTok, nt = m - t0 < kTok ? m - t0 : kTok;
-    const int tid = (int)threadIdx.x, lane = tid & 63, n = lane & 15, b = lane >> 4;
+// Up to 8 rows of bf16 weights bound by HBM (128256 x 2560, 657 MB: 101 to
+// 107 us, 6.4 TB/s; lmhead_batch_kernel 143), beyond and for int8 weights by
+// the f32 multiply-adds (68 us per 16 rows, used or not, 51 per 12) with the widening
+// after them: matrix and vector instructions take turns on a SIMD.  bf16, 16
+// rows 199 -> 132 us, 24 rows 372 -> 215, 64 rows 756 -> 488; int8, 6 rows 129 ->
+// 88, 16 rows 189 -> 132, 24 rows 359 -> 206.  Measured beside it: 16 x 16 x 1 instructions (four
+// chains), with the token rows in LDS and a whole tile a wavefront (16 rows of
+// bf16 160 us, with 64-byte pieces of a row a load 200), and with the chains
+// split over eight wavefronts, token rows in registers and an exchange of the
+// sums through LDS (150; 64 rows 477).
+template <int NCH, bool FULL, bool Q8, int TG, int RG, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void lmhead_tile_kernel(
+    const void* W, const float* rscale, int rows, int cols, const float* xn, int m, int part_tiles, float* logits,
+    unsigned long long* key) {
+    constexpr int G = NCH * 128;  // 16-byte granules per token row
+    constexpr int STEPS = 4 * NCH, RING = RG == 2 ? 2 * NCH : TG == 3 && !Q8 ? 2 : 4, NW = NT / 64;  // | STEPS
+    constexpr int RT = 4 * RG;  // weight rows per wavefront and tile
+    using Chunk = typename std::conditional<Q8, u32x2, u32x4>::type;
+    extern __shared__ __align__(16) float xs[];  // [4 TG][4 G]
+    const int tid = (int)threadIdx.x, lane = tid & 63, j = lane & 3, k = lane >> 2;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nchunks = cols >> 3, c0 = 8 * w + 2 * b;  // this lane's chunks: c0 + a + 64 i
-    const int ntiles = (rows + kVoc - 1) / kVoc;
+    const int nchunks = cols >> 3, ntiles = (rows + RT - 1) / RT;
+    const int ngroups = (m + 4 * TG - 1) / (4 * TG), ntw = (int)gridDim.x / ngroups;
+    const int t0 = (int)blockIdx.x / ntw * (4 * TG), part = (int)blockIdx.x % ntw;
+    const int nt = m - t0 < 4 * TG ? m - t0 : 4 * TG;
+    xn += (size_t)t0 * cols;
     const int tile_end = (part + 1) * part_tiles < ntiles ? (part + 1) * part_tiles : ntiles;
+    constexpr int kG[4] = {0, 2, 1, 3};
 
-    u32x4 wb[2][NCH][NV];
-    auto load = [&](int tile, int i, u32x4 (&d)[NV]) {
-        int r = tile * kVoc + n;
-        r = r < rows ? r : rows - 1;  // past the end: a valid row (not stored)
-        const char* p = (const char*)W + (size_t)r * cols * (Q8 ? 1 : 2);
-        const bool all = FULL || i + 1 < NCH;  // only a last chunk can be past the row's end
-        const int c = c0 + 64 * i;
-        if constexpr (Q8) {
-            if (FULL) {
-                d[0] = __builtin_nontemporal_load((const LBT_GLOBAL u32x4*)(p + 8 * c));
-            } else if (all) {  // rows are multiples of 8 bytes: two 8-byte loads
-                d[0].xy = __builtin_nontemporal_load((const LBT_GLOBAL u32x2*)(p + 8 * c));
-                d[0].zw = __builtin_nontemporal_load((const LBT_GLOBAL u32x2*)(p + 8 * c + 8));
-            } else {
-                d[0] = u32x4{0, 0, 0, 0};
-                if (c < nchunks) d[0].xy = __builtin_nontemporal_load((const LBT_GLOBAL u32x2*)(p + 8 * c));
-                if (c + 1 < nchunks) d[0].zw = __builtin_nontemporal_load((const LBT_GLOBAL u32x2*)(p + 8 * c + 8));
-            }
-        } else {
+    // step s: chunks 16 g + k + 64 i of 16 rows, g = kG[s / NCH], i = s % NCH
+    Chunk wb[RING][RG];
+    auto load = [&](int tile, int s, Chunk (&d)[RG]) {
+        const int i = s % NCH, c = 16 * kG[s / NCH] + k + 64 * i;
 #pragma unroll
-            for (int a = 0; a < 2; a++) {
-                if (!all) d[a] = u32x4{0, 0, 0, 0};
-                if (all || c + a < nchunks)
-                    d[a] = __builtin_nontemporal_load((const LBT_GLOBAL u32x4*)(p + 16 * (c + a)));
-            }
+        for (int rg = 0; rg < RG; rg++) {
+            int r = tile * RT + 4 * rg + j;
+            r = r < rows ? r : rows - 1;  // past the end: a valid row (not stored)
+            const Chunk* p = (const Chunk*)((const char*)W + (size_t)r * cols * (Q8 ? 1 : 2)) + c;
+            d[rg] = Chunk{};
+            if (FULL || i + 1 < NCH || c < nchunks)  // only a last chunk can be past the row's end
+                d[rg] = __builtin_nontemporal_load((const LBT_GLOBAL Chunk*)p);
         }
     };
-    int tile = part * part_tiles;
-    if (tile >= tile_end) return;  // (the whole workgroup)
+    int tile = part * part_tiles + w;
+    const int first = tile < tile_end ? tile : 0;
 #pragma unroll
-    for (int k = 0; k < 2; k++)
-#pragma unroll
-        for (int i = 0; i < NCH; i++) load(tile + k, i, wb[k][i]);
+    for (int s = 0; s < RING; s++) load(first, s, wb[s]);
 
-    // this lane's token row; columns past the end are -0: its product with a
-    // zero weight leaves every sum as it is
-    float xv[NCH][2][8];
-#pragma unroll
-    for (int i = 0; i < NCH; i++)
-#pragma unroll
-        for (int a = 0; a < 2; a++) {
-            const int c = c0 + a + 64 * i;
-            const float* p = xn + (size_t)(t0 + (n < nt ? n : 0)) * cols + 8 * c;
-            const bool in = FULL || i + 1 < NCH || c < nchunks;
-            if (((uintptr_t)xn & 15) == 0) {  // uniform
-                const f32x4 pad = {-0.0f, -0.0f, -0.0f, -0.0f};
-                const f32x4 lo = in ? gload((const f32x4*)p) : pad, hi = in ? gload((const f32x4*)p + 1) : pad;
-#pragma unroll
-                for (int e = 0; e < 4; e++) xv[i][a][e] = lo[e], xv[i][a][4 + e] = hi[e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) xv[i][a][e] = in ? gload(p + e) : -0.0f;
-            }
+    // token rows; columns past the end are -0: a product of it with a zero
+    // weight leaves every sum as it is
+    auto swz = [](int t) { return (t & 1) + 4 * (t & 2); };
+    if (cols == 4 * G && ((uintptr_t)xn & 15) == 0) {
+        for (int i = tid; i < 4 * TG * G; i += NT) {
+            const int t = i / G, g = i % G;
+            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (t < nt) v = gload((const f32x4*)(xn + (size_t)t * cols) + g);
+            *(f32x4*)(xs + 4 * (t * G + (g ^ swz(t)))) = v;
         }
+    } else {
+        for (int i = tid; i < 4 * TG * G * 4; i += NT) {
+            const int t = i / (4 * G), e = i % (4 * G);
+            float v = -0.0f;
+            if (t < nt && e < cols) v = gload(xn + (size_t)t * cols + e);
+            xs[4 * (t * G + ((e >> 2) ^ swz(t))) + (e & 3)] = v;
+        }
+    }
+    __syncthreads();
+    const float* xa[TG][2];  // this lane's token row (j of each group), halves of chunk k
+#pragma unroll
+    for (int tg = 0; tg < TG; tg++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) xa[tg][h] = xs + 4 * ((4 * tg + j) * G + ((2 * k + h) ^ swz(j)));
 
-    // this lane's output after the exchange: registers 4 blk + oi of lane ol
-    const int oi = w >> 1, ol = (w & 1) * 32 + (lane & 31), oa = lane >> 5;
-    const int otok = 4 * (ol >> 4) + oi, ovoc = ol & 15;
-    unsigned long long best = 0ull;
+    // this lane's outputs after the halving: sums NS k .. of the 4 RG TG of a
+    // weight row j, sum index (token group * RG + row group) * 4 + token
+    constexpr int NS = TG * RG / 4;
+    const int i0 = NS * k;
+    auto orow = [&](int z) { return 4 * (((i0 + z) >> 2) % RG) + j; };
+    auto otok = [&](int z) { return 4 * (((i0 + z) >> 2) / RG) + ((i0 + z) & 3); };
+    unsigned long long best[NS] = {};
 
-    // the chains of this lane's output, read ahead of the next tile's work and added after it
-    float pv[4][8];
-    auto fetch = [&](const float* buf) {
-        __syncthreads();
-        const float* pr = buf + (oa * 16 + oi) * 64 + ol;
+    for (; tile < tile_end; tile += NW) {
+        f32x4 c[TG][RG], a[TG][RG], t[TG][RG];  // current g; g 0 (+ 2); g 1
+        const int next = tile + NW < tile_end ? tile + NW : tile;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int s = 0; s < STEPS; s++) {
+            Chunk (&cur)[RG] = wb[s % RING];
+            const int i = s % NCH, gs = s / NCH;
 #pragma unroll
-            for (int q = 0; q < 8; q++) pv[k][q] = pr[(q * 32 + 4 * k) * 64];
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // the wavefront's chains of a tile; the slots reload for the tile after the next
-    auto chains = [&](int tile, u32x4 (&d)[NCH][NV], f32x16 (&c)[2], const float* prev) {
+            for (int rg = 0; rg < RG; rg++) pin(cur[rg]);
+            float xv[TG][8];
 #pragma unroll
-        for (int i = 0; i < NCH; i++) {
-            if (i == NCH / 2 && prev) fetch(prev);  // the previous tile's sums: the barrier falls amid this tile's work
+            for (int tg = 0; tg < TG; tg++)
 #pragma unroll
-            for (int v = 0; v < NV; v++) pin(d[i][v]);
+                for (int h = 0; h < 2; h++) {
+                    const f32x4 v = *(const f32x4*)(xa[tg][h] + 4 * (32 * kG[gs] + 128 * i));
 #pragma unroll
-            for (int a = 0; a < 2; a++) {
+                    for (int e = 0; e < 4; e++) xv[tg][4 * h + e] = v[e];
+                }
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++) {
                 float wf[8];
                 if constexpr (Q8) {
-                    // byte ^ 0x80 is the weight + 128; as the low byte of 2^23's
-                    // mantissa it is 2^23 + 128 + weight, the subtraction exact
 #pragma unroll
                     for (int e = 0; e < 8; e++)
-                        wf[e] = __uint_as_float(__builtin_amdgcn_perm(0x4b000000u,
-                                                                      d[i][0][2 * a + (e >> 2)] ^ 0x80808080u,
+                        wf[e] = __uint_as_float(__builtin_amdgcn_perm(0x4b000000u, cur[rg][e >> 2] ^ 0x80808080u,
                                                                       0x07040400u + (e & 3))) -
                                 8388736.0f;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        wf[2 * e] = __uint_as_float(d[i][a][e] << 16);
-                        wf[2 * e + 1] = __uint_as_float(d[i][a][e] & 0xffff0000u);
+                        wf[2 * e] = __uint_as_float(cur[rg][e] << 16);
+                        wf[2 * e + 1] = __uint_as_float(cur[rg][e] & 0xffff0000u);
                     }
                 }
 #pragma unroll
-                for (int e = 0; e < 8; e++) c[a] = outer4(xv[i][a][e], wf[e], i == 0 && e == 0 ? f32x16{} : c[a]);
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int tg = 0; tg < TG; tg++)
+                        c[tg][rg] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                            xv[tg][e], wf[e], i == 0 && e == 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : c[tg][rg], 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            load(tile + 2, i, d[i]);
+            load(s + RING < STEPS ? tile : next, (s + RING) % STEPS, cur);
+            if (i == NCH - 1) {
+#pragma unroll
+                for (int tg = 0; tg < TG; tg++)
+#pragma unroll
+                    for (int rg = 0; rg < RG; rg++) {
+                        if (gs == 0) a[tg][rg] = c[tg][rg];
+                        else if (gs == 1) a[tg][rg] = a[tg][rg] + c[tg][rg];
+                        else if (gs == 2) t[tg][rg] = c[tg][rg];
+                        else a[tg][rg] = a[tg][rg] + (t[tg][rg] + c[tg][rg]);
+                        if (gs != 2) pin(a[tg][rg]);
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    auto publish = [&](const f32x16 (&c)[2], float* buf) {
-        float* pw = buf + (size_t)w * 2 * 16 * 64 + lane;
+        float v[TG * RG * 4], o[NS];
 #pragma unroll
-        for (int a = 0; a < 2; a++)
+        for (int tg = 0; tg < TG; tg++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) pw[(a * 16 + r) * 64] = c[a][r];
-    };
-    auto finish = [&](int tile) {
-        float blk[4];
+            for (int rg = 0; rg < RG; rg++)
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            blk[k] = ((pv[k][0] + pv[k][4]) + (pv[k][2] + pv[k][6])) + ((pv[k][1] + pv[k][5]) + (pv[k][3] + pv[k][7]));
-        float sum = xor_add<32>((blk[0] + blk[2]) + (blk[1] + blk[3]));
-        const int row = tile * kVoc + ovoc;
-        if (oa == 0 && otok < nt && row < rows) {
-            if constexpr (Q8) sum = gload(rscale + row) * sum;
-            if (logits) gstore(logits + (size_t)(t0 + otok) * rows + row, sum);
-            const unsigned long long k = argmax_key(sum, (uint32_t)row);
-            best = k > best ? k : best;
+                for (int e = 0; e < 4; e++) v[(tg * RG + rg) * 4 + e] = a[tg][rg][e];
+        {
+            float h1[TG * RG * 2], h2[TG * RG], h3[TG * RG / 2];
+            halve<32>(v, h1);
+            halve<16>(h1, h2);
+            halve<8>(h2, h3);
+            halve<4>(h3, o);
         }
-    };
-    // one barrier a tile: a buffer is written again two tiles later, past the
-    // barrier that follows its readers' adds
-    float* const buf0 = part_s;
-    float* const buf1 = part_s + 8 * 2 * 16 * 64;
-    f32x16 c[2];
-    chains(tile, wb[0], c, nullptr);
-    publish(c, buf0);
-    for (; tile + 2 < tile_end; tile += 2) {
-        chains(tile + 1, wb[1], c, buf0);
-        finish(tile);
-        publish(c, buf1);
-        chains(tile + 2, wb[0], c, buf1);
-        finish(tile + 1);
-        publish(c, buf0);
+#pragma unroll
+        for (int z = 0; z < NS; z++) {
+            const int row = tile * RT + orow(z);
+            if (row >= rows || otok(z) >= nt) continue;
+            const float sum = Q8 ? gload(rscale + row) * o[z] : o[z];
+            if (logits) gstore(logits + (size_t)(t0 + otok(z)) * rows + row, sum);
+            const unsigned long long kz = argmax_key(sum, (uint32_t)row);
+            best[z] = kz > best[z] ? kz : best[z];
+        }
     }
-    const float* last = buf0;
-    if (tile + 1 < tile_end) {
-        chains(tile + 1, wb[1], c, buf0);
-        finish(tile);
-        publish(c, buf1);
-        tile++;
-        last = buf1;
-    }
-    fetch(last);
-    finish(tile);
 #pragma unroll
-    for (int k = 0; k < 2; k++)
+    for (int s = 0; s < RING; s++)
 #pragma unroll
-        for (int i = 0; i < NCH; i++)
-#pragma unroll
-            for (int v = 0; v < NV; v++) keep(wb[k][i][v]);
+        for (int rg = 0; rg < RG; rg++) keep(wb[s][rg]);
     if (!key) return;
-    // one atomic per (workgroup, token): lanes 16 apart hold different tokens
-    unsigned long long k = best;
+    // one atomic per (workgroup, token): the lanes' keys meet in LDS once
+    // every wavefront is done with the token rows
+    __syncthreads();
+    unsigned long long* wbest = (unsigned long long*)xs;  // [4 TG][NW][KW]
+    constexpr int KW = RT;  // keys per wavefront and token
 #pragma unroll
-    for (int d = 8; d >= 1; d >>= 1) {
-        const unsigned long long o = __shfl_xor(k, d);
-        k = o > k ? o : k;
+    for (int z = 0; z < NS; z++) wbest[otok(z) * (NW * KW) + w * KW + orow(z)] = best[z];
+    __syncthreads();
+    if (tid < nt) {
+        unsigned long long b = 0ull;
+        for (int i = 0; i < NW * KW; i++) b = wbest[tid * (NW * KW) + i] > b ? wbest[tid * (NW * KW) + i] : b;
+        if (b) atomicMax(&key[t0 + tid], b);
     }
-    if (oa == 0 && ovoc == 0 && otok < nt && k) atomicMax(&key[t0 + otok], k);
 }
 
 namespace {
 
-template <int NCH, bool FULL, bool Q8>
-int launch(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int cols, const float* xn, int m,
-           float* logits, unsigned long long* key) {
-    constexpr size_t lds = (size_t)2 * 8 * 2 * 16 * 64 * 4;
+template <int NCH, bool FULL, bool Q8, int TG, int RG, int NT>
+int launch_tile(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int cols, const float* xn, int m,
+                float* logits, unsigned long long* key) {
+    constexpr size_t lds = (size_t)4 * TG * NCH * 128 * 16;
     // on every call: per device, and without state of ours
-    LBT_HIP(ctx, hipFuncSetAttribute((const void*)lmhead_tile_kernel<NCH, FULL, Q8>,
+    LBT_HIP(ctx, hipFuncSetAttribute((const void*)lmhead_tile_kernel<NCH, FULL, Q8, TG, RG, NT>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int ngroups = (m + kTok - 1) / kTok, ntiles = (rows + kVoc - 1) / kVoc;
-    int parts = ctx->cus / ngroups;
+    const int ngroups = (m + 4 * TG - 1) / (4 * TG), ntiles = (rows + 4 * RG - 1) / (4 * RG);
+    int parts = (NT == kThreads ? 2 : 1) * ctx->cus / ngroups;
     if (parts < 1) parts = 1;
     const int part_tiles = (ntiles + parts - 1) / parts;
     parts = (ntiles + part_tiles - 1) / part_tiles;
     hipEvent_t e0, e1;
     prof_pair(ctx, &e0, &e1);
-    hipExtLaunchKernelGGL((lmhead_tile_kernel<NCH, FULL, Q8>), dim3(parts * ngroups), dim3(kNT), lds, ctx->stream, e0,
-                          e1, 0, w, rscale, rows, cols, xn, m, part_tiles, logits, key);
+    hipExtLaunchKernelGGL((lmhead_tile_kernel<NCH, FULL, Q8, TG, RG, NT>), dim3(parts * ngroups), dim3(NT), lds,
+                          ctx->stream, e0, e1, 0, w, rscale, rows, cols, xn, m, part_tiles, logits, key);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_err(ctx, e, "lmhead_tile_kernel launch");
     prof_commit(ctx, e0, e1, kProfHead, (double)rows * cols * (Q8 ? 1.0 : 2.0));
     return LBT_OK;
+}
+template <int NCH, bool FULL, bool Q8>
+int launch_tg(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int cols, const float* xn, int m,
+              float* logits, unsigned long long* key) {
+    if (m <= 4) return launch_tile<NCH, FULL, Q8, 1, 4, kThreads>(ctx, w, rscale, rows, cols, xn, m, logits, key);
+    if (m <= 8) return launch_tile<NCH, FULL, Q8, 2, 4, kThreads>(ctx, w, rscale, rows, cols, xn, m, logits, key);
+    // 12 token rows a workgroup where that takes no more groups than 16 (9 to
+    // 12, 17 to 24, 33 to 36 rows): 128256 x 2560, 24 rows bf16 245 -> 215 us,
+    // int8 248 -> 206; 9 rows 135 -> 122 and 130 -> 107
+    if ((m + 11) / 12 == (m + 15) / 16)
+        return launch_tile<NCH, FULL, Q8, 3, 4, 512>(ctx, w, rscale, rows, cols, xn, m, logits, key);
+    return launch_tile<NCH, FULL, Q8, 4, 2, 512>(ctx, w, rscale, rows, cols, xn, m, logits, key);
 }
 
 }  // namespace
@@ -270,20 +264,21 @@ int launch_head_tile(lbt_ctx* ctx, const void* w, const float* rscale, int rows,
     const int nch = (cols / 8 + 63) / 64;
     if (cols % 8 || cols <= 0 || rows <= 0 || m < 1 || nch > kMaxNch) return 1;
     const bool full = cols % 512 == 0;
-    // Up to 8 rows lmhead_batch_kernel's 8-row groups waste nothing: it stays
-    // where columns past a chain's last chunk would have to be masked (1000
-    // columns x 32000 rows, 6 rows of int8: 22.3 against 25.8 us), and so it does
-    // with fewer than two tiles a CU (2560 x 4000: 11 against 17 us at 6 rows, 15
-    // to 17 against 19 at 16).
-    const long tiles = (long)((rows + kVoc - 1) / kVoc) * ((m + kTok - 1) / kTok);
-    if ((m <= 8 && !full) || tiles <= 2L * ctx->cus) return 1;
-#define LBT_HEAD_TILE(N)                                                                                \
-    case N:                                                                                             \
-        if (rscale)                                                                                     \
-            return full ? launch<N, true, true>(ctx, w, rscale, rows, cols, xn, m, logits, key)         \
-                        : launch<N, false, true>(ctx, w, rscale, rows, cols, xn, m, logits, key);       \
-        return full ? launch<N, true, false>(ctx, w, nullptr, rows, cols, xn, m, logits, key)           \
-                    : launch<N, false, false>(ctx, w, nullptr, rows, cols, xn, m, logits, key);
+    // Every workgroup first stages its token rows (80 KB at 8 rows of 2560
+    // columns): matrices of fewer than two 16-row tiles a CU, four at 5 to 8
+    // rows, stay on lmhead_batch_kernel (2560 x 4000: 12 against 13 us at 2
+    // rows, 12 against 18 at 8, 17 against 19 at 9; 2560 x 9000: 23 against 18
+    // at 2, 23 against 25 at 8, 34 against 25 at 9; 2560 x 24000 at 8: 40
+    // against 30).
+    const long tiles = (long)((rows + 15) / 16) * ((m + 15) / 16);
+    if (tiles <= (m > 4 && m <= 8 ? 4L : 2L) * ctx->cus) return 1;
+#define LBT_HEAD_TILE(N)                                                                             \
+    case N:                                                                                          \
+        if (rscale)                                                                                  \
+            return full ? launch_tg<N, true, true>(ctx, w, rscale, rows, cols, xn, m, logits, key)   \
+                        : launch_tg<N, false, true>(ctx, w, rscale, rows, cols, xn, m, logits, key); \
+        return full ? launch_tg<N, true, false>(ctx, w, nullptr, rows, cols, xn, m, logits, key)     \
+                    : launch_tg<N, false, false>(ctx, w, nullptr, rows, cols, xn, m, logits, key);
     switch (nch) {
         LBT_HEAD_TILE(1)
         LBT_HEAD_TILE(2)

@@ -34,8 +34,8 @@ def linear_dev(ctx, fn, h, x, rows, offset=0):
 
 # rows: whole and ragged 16-row tiles, few and many a CU, an odd and an even
 # number a workgroup; cols: one to five chunks a chain, whole and cut
-@pytest.mark.parametrize("rows,cols", [(9001, 8), (9001, 128), (12345, 512), (8209, 520), (9000, 1000), (8300, 1536),
-                                       (9007, 2040), (8200, 2552), (16400, 2560), (24577, 2560)])
+@pytest.mark.parametrize("rows,cols", [(16401, 8), (16409, 128), (17345, 512), (16399, 520), (18000, 1000),
+                                       (16500, 1536), (16807, 2040), (16392, 2552), (16400, 2560), (24577, 2560)])
 @pytest.mark.parametrize("q8", [False, True])
 def test_several_rows_equal_one_row(ctx, rows, cols, q8):
     rng = np.random.default_rng(rows + cols)
@@ -50,7 +50,7 @@ def test_several_rows_equal_one_row(ctx, rows, cols, q8):
     x[5] *= 1e-20  # with the small rows: products below the denormals
     x[7] = 0.0
     one = np.concatenate([linear_dev(ctx, fn, h.h, x[i:i + 1], rows) for i in range(50)])
-    for m, offset in ((2, 0), (9, 0), (16, 1), (17, 0), (33, 3), (50, 0)):
+    for m, offset in ((2, 0), (4, 1), (5, 0), (8, 0), (9, 0), (12, 1), (13, 0), (16, 1), (17, 0), (24, 2), (33, 3), (50, 0)):
         announce(f"head rows={rows} cols={cols} q8={q8} m={m} offset={offset}")
         got = linear_dev(ctx, fn, h.h, x[:m], rows, offset)
         assert np.array_equal(got.view(np.uint32), one[:m].view(np.uint32)), m
