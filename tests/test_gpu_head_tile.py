@@ -33,8 +33,10 @@ def linear_dev(ctx, fn, h, x, rows, offset=0):
 
 
 # rows: whole and ragged 16-row tiles, few and many a CU, an odd and an even
-# number a workgroup; cols: one to five chunks a chain, whole and cut
-@pytest.mark.parametrize("rows,cols", [(16401, 8), (16409, 128), (17345, 512), (16399, 520), (18000, 1000),
+# number a workgroup; cols: one to five chunks a chain, whole and cut; first
+# matrices that stay on the older kernels
+@pytest.mark.parametrize("rows,cols", [(300, 8), (1001, 648), (4000, 2560), (16401, 8), (16409, 128),
+                                       (17345, 512), (16399, 520), (18000, 1000),
                                        (16500, 1536), (16807, 2040), (16392, 2552), (16400, 2560), (24577, 2560)])
 @pytest.mark.parametrize("q8", [False, True])
 def test_several_rows_equal_one_row(ctx, rows, cols, q8):
