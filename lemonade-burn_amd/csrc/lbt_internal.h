@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/lbt.h"
+#include "rules.h"
 
 // Path selection read once from the environment when a context is created
 // (lbt_ctx_create); measurements and tests choose a path per context.

@@ -205,16 +205,17 @@ __device__ __forceinline__ void mfma_epilogue(const GemvArgs& a, AccT (&acc)[MS]
 }
 
 // The same values for a wavefront block whose rows all lie in one matrix (or
-// past its end): no per-store bounds branch (tokens past M fall outside the
-// stores' buffer, rows past the end are masked once per row tile), one
-// division per token (the per-row-block scale is the block's one matrix
-// scale), 32-bit offsets from the matrix's base (the compiler then uses
-// scalar-base stores), the residual's old values loaded half a tile ahead of
-// its stores.  TAIL: the block reaches past the last row.  A prompt is rarely a multiple of the tile, and the launch lasts
-// as long as its ragged tiles: with those on the general epilogue the q/k/v
-// GEMM of 3000 tokens of the 2B shape took 134 us, now 69.  Instruction count, not
-// memory, bounds the epilogue of a 128 x 128 tile (2088 instructions per
-// wavefront in the general form).
+// past its end) and whose offsets fit 32 bits (epi32_takes): no per-store
+// bounds branch (tokens past M fall outside the stores' buffer, rows past the
+// end are masked once per row tile), one division per token (the
+// per-row-block scale is the block's one matrix scale), 32-bit offsets from
+// the matrix's base (the compiler then uses scalar-base stores), the
+// residual's old values loaded half a tile ahead of its stores.  TAIL: the
+// block reaches past the last row.  A prompt is rarely a multiple of the
+// tile, and the launch lasts as long as its ragged tiles: with those on the
+// general epilogue the q/k/v GEMM of 3000 tokens of the 2B shape took 134 us,
+// now 69.  Instruction count, not memory, bounds the epilogue of a 128 x 128
+// tile (2088 instructions per wavefront in the general form).
 // Per-token values of a wavefront block's 32 MS tokens: lane j holds token
 // tok0 + j's sum(q) and 1/(s_a*s_w) of matrix mt (one load pair and one
 // division per lane, instead of one per lane and D-tile element); the
@@ -252,7 +253,8 @@ __device__ __forceinline__ void epi32_pre(const GemvArgs& a, int tok0, float swm
 
 // Whether a wavefront block takes a lean epilogue; its matrix, first row and
 // scale.  Unpaired outputs: its rows in one matrix.  q/k/v: whole, in one
-// matrix.  Gate/up: whole.  32-bit byte offsets of the output.
+// matrix.  Gate/up: whole.  32-bit byte offsets of the output, those of the
+// block's tokens past M included (lean_offsets_fit).
 template <int OUT, int MS, int NS>
 __device__ __forceinline__ bool epi32_takes(const GemvArgs& a, int tok0, int row0, int& mt0, int& ro0, float& swm) {
     const int end = row0 + NS * 32, total = a.total_rows;
@@ -261,7 +263,7 @@ __device__ __forceinline__ bool epi32_takes(const GemvArgs& a, int tok0, int row
         mt0 = 0;
         ro0 = row0 >> 1;
         swm = a.sw[0];
-        return end <= total && (long)a.m * a.rows[0] < (1L << 30);
+        return end <= total && lean_offsets_fit(a.m, a.rows[0], tok0, MS * 32, NS * 32);
     }
     int mt1, ro1;
     resolve_row<OUT>(a, row0, mt0, ro0);
@@ -269,7 +271,7 @@ __device__ __forceinline__ bool epi32_takes(const GemvArgs& a, int tok0, int row
     swm = mt0 == 0 ? a.sw[0] : (mt0 == 1 ? a.sw[1] : a.sw[2]);
     if constexpr (OUT == kOutQKV) return end <= total && mt0 == mt1;
     const int ldm = mt0 == 0 ? a.rows[0] : (mt0 == 1 ? a.rows[1] : a.rows[2]);
-    return mt0 == mt1 && (long)a.m * ldm < (1L << 30);
+    return mt0 == mt1 && lean_offsets_fit(a.m, ldm, tok0, MS * 32, NS * 32);
 }
 
 template <int OUT, int MS, int NS, bool TAIL>
@@ -283,8 +285,8 @@ __device__ __forceinline__ void epi32_full(const GemvArgs& a, v16i (&acc)[MS][NS
     const int ld = mt == 0 ? a.rows[0] : (mt == 1 ? a.rows[1] : a.rows[2]);
     void* const outv = mt == 0 ? a.out[0] : (mt == 1 ? a.out[1] : a.out[2]);
     // stores through a buffer resource: the matrix base in scalar registers,
-    // a 32-bit byte offset per lane (the caller checks M * ld < 2^30); tokens
-    // past M are past its end
+    // a 32-bit byte offset per lane; tokens past M are past its end (the
+    // caller checks that none of the block's offsets wraps, lean_offsets_fit)
     const __amdgpu_buffer_rsrc_t ob = buf_rsrc(outv, (uint32_t)a.m * (uint32_t)ld * 4u);
 #pragma unroll
     for (int ms = 0; ms < MS; ms++) {
