@@ -1113,12 +1113,8 @@ int launch_head(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int 
                                    : (const void*)lmhead_batch_kernel<kR, kLmChunks, 16, false, 512>)
                              : (q8 ? (const void*)lmhead_batch_kernel<kR, kLmChunks, kTG, true>
                                    : (const void*)lmhead_batch_kernel<kR, kLmChunks, kTG, false>);
-        static bool attr[4] = {false, false, false, false};
-        if (!attr[q8 + 2 * big]) {
-            (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, big ? 160 * 1024 : 96 * 1024);
-            (void)hipGetLastError();
-            attr[q8 + 2 * big] = true;
-        }
+        // on every call: per device, and without state of ours
+        LBT_HIP(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, big ? 160 * 1024 : 96 * 1024));
         if (lds > (big ? 160 : 96) * 1024)
             return set_err(ctx, LBT_E_INVALID, std::string(what) + ": token group exceeds LDS");
         hipEvent_t e0, e1;

@@ -1124,16 +1124,7 @@ namespace {
 template <int MS, int NS, int KB, int ST = kG2Stages>
 hipError_t launch_tiles2(const GemvArgs& a, int out_mode, dim3 grid, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     constexpr size_t lds = (size_t)ST * (64 * MS) * (128 * KB);
-    static bool attr = false;
-    if (!attr) {
-        const void* fns[] = {(const void*)tgemm2_kernel<kOutI32, MS, NS, KB, ST>, (const void*)tgemm2_kernel<kOutF32, MS, NS, KB, ST>,
-                             (const void*)tgemm2_kernel<kOutF32Add, MS, NS, KB, ST>,
-                             (const void*)tgemm2_kernel<kOutRelu2, MS, NS, KB, ST>,
-                             (const void*)tgemm2_kernel<kOutQKV, MS, NS, KB, ST>};
-        for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        (void)hipGetLastError();
-        attr = true;
-    }
+    static_assert(lds <= 64 * 1024, "more needs the kernel's LDS limit raised on every call");
     switch (out_mode) {
         case kOutI32: hipExtLaunchKernelGGL((tgemm2_kernel<kOutI32, MS, NS, KB, ST>), grid, dim3(kThreads), lds, s, e0, e1, 0, a); break;
         case kOutF32: hipExtLaunchKernelGGL((tgemm2_kernel<kOutF32, MS, NS, KB, ST>), grid, dim3(kThreads), lds, s, e0, e1, 0, a); break;
@@ -1149,17 +1140,7 @@ template <int WM, int WN, int MS, int NS, int KB, int ST>
 hipError_t launch_tiles3(const GemvArgs& a, int out_mode, dim3 grid, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     constexpr int NT = 64 * WM * WN;
     constexpr size_t lds = (size_t)ST * (32 * MS * WM) * (128 * KB);
-    static bool attr = false;
-    if (!attr) {
-        const void* fns[] = {(const void*)tgemm3_kernel<kOutI32, WM, WN, MS, NS, KB, ST>,
-                             (const void*)tgemm3_kernel<kOutF32, WM, WN, MS, NS, KB, ST>,
-                             (const void*)tgemm3_kernel<kOutF32Add, WM, WN, MS, NS, KB, ST>,
-                             (const void*)tgemm3_kernel<kOutRelu2, WM, WN, MS, NS, KB, ST>,
-                             (const void*)tgemm3_kernel<kOutQKV, WM, WN, MS, NS, KB, ST>};
-        for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        (void)hipGetLastError();
-        attr = true;
-    }
+    static_assert(lds <= 64 * 1024, "more needs the kernel's LDS limit raised on every call");
     switch (out_mode) {
         case kOutI32: hipExtLaunchKernelGGL((tgemm3_kernel<kOutI32, WM, WN, MS, NS, KB, ST>), grid, dim3(NT), lds, s, e0, e1, 0, a); break;
         case kOutF32: hipExtLaunchKernelGGL((tgemm3_kernel<kOutF32, WM, WN, MS, NS, KB, ST>), grid, dim3(NT), lds, s, e0, e1, 0, a); break;

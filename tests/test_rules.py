@@ -1,6 +1,7 @@
 """The conditions of csrc/rules.h, compiled for the CPU: what a path is
 chosen by, checked against what the path does with the sizes."""
 import ctypes as C
+import re
 import subprocess
 from pathlib import Path
 
@@ -58,3 +59,12 @@ def test_lean_epilogue_keeps_the_blocks_it_can_address(rules):
     for m, ld in ((33, 3840), (301, 1706), (3000, 13824), (2048, 2560), (8000, 128256)):
         for tok0 in range(0, m, 64):
             assert rules.lean_offsets_fit(m, ld, tok0, 64, 64)
+
+
+def test_no_launch_keeps_per_process_state():
+    # A kernel's LDS limit belongs to the device the context is on: a flag set
+    # once per process leaves a second device without it, and races between
+    # threads.  Launch code holds no writable function-level statics.
+    for src in sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp")):
+        for n, line in enumerate(src.read_text().splitlines(), 1):
+            assert not re.match(r"\s+static (?!const|inline|_)", line), f"{src.name}:{n}: {line.strip()}"
