@@ -1082,20 +1082,23 @@ int launch_head(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int 
     if (m <= 0) return LBT_OK;
     constexpr int kTG = 8, kR = 4;
     const double wbytes = (double)rows * cols * (q8 ? 1.0 : 2.0);
-    if (m >= 2 && (xn || !norm_w) && cols <= 64 * kLmChunks * 8) {
+    const bool choose = !ctx->tune.head_tg8 && !ctx->tune.head_batch_classic;  // the switches force their kernels
+    const bool several = m >= 2 && (xn || !norm_w) && cols <= 64 * kLmChunks * 8 &&
+                         !(choose && !norm_w && head_row_by_row(rows, cols, m, q8, ctx->cus));
+    if (several) {
         // several rows: normalize once, then a weight-reusing head
         if (norm_w) {
             hipLaunchKernelGGL(row_norm_kernel, dim3(m), dim3(kThreads), 0, ctx->stream, x, cols, norm_w, eps, xn);
             LBT_HIP(ctx, hipGetLastError());
             x = xn;
         }
-        if (!ctx->tune.head_tg8 && !ctx->tune.head_batch_classic) {
+        if (choose) {
             const int rc = launch_head_tile(ctx, w, rscale, rows, cols, x, m, logits, key);
             if (rc != 1) return rc;
         }
     }
-    if (m >= 2 && (xn || !norm_w) && cols <= 64 * kLmChunks * 8 && ((uintptr_t)x & 15) == 0) {
-        // small matrices (launch_head_tile's rule), and the switches;
+    if (several && ((uintptr_t)x & 15) == 0) {
+        // small matrices (head_tiled), and the switches;
         // more than 8 rows: 16-token groups on 512 threads (the whole LDS of a
         // CU; each weight row is then read from L2 half as often), else
         // 8-token groups on 256 threads (two workgroups per CU)

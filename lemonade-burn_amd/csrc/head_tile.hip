@@ -264,16 +264,7 @@ int launch_head_tile(lbt_ctx* ctx, const void* w, const float* rscale, int rows,
     const int nch = (cols / 8 + 63) / 64;
     if (cols % 8 || cols <= 0 || rows <= 0 || m < 1 || nch > kMaxNch) return 1;
     const bool full = cols % 512 == 0;
-    // Every workgroup first stages its token rows (80 KB at 8 rows of 2560
-    // columns): matrices of fewer than two 16-row tiles a CU, four at 5 to 8
-    // rows, stay on the older kernels (lmhead_batch_kernel, 2560 x 4000: 12
-    // against 13 us at 2 rows, 12 against 18 at 8; 2560 x 9000: 23 against 18
-    // at 2, 23 against 25 at 8; 2560 x 24000 at 8: 40 against 30;
-    // lmhead_stream_kernel, 16 rows, 2560 x 4000: 13 against 20, x 8500: 25
-    // against 26, x 12300: 31 against 28; 24 rows, x 4000: 20 against 21, x
-    // 8500: 37 against 31).
-    const long tiles = (long)((rows + 15) / 16) * ((m + 15) / 16);
-    if (tiles <= (m > 4 && m <= 8 ? 4L : 2L) * ctx->cus) return 1;
+    if (!head_tiled(rows, m, ctx->cus)) return 1;
 #define LBT_HEAD_TILE(N)                                                                             \
     case N:                                                                                          \
         if (rscale)                                                                                  \

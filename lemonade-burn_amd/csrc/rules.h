@@ -16,4 +16,39 @@ constexpr bool lean_offsets_fit(int64_t m, int64_t ld, int64_t tok0, int64_t tok
     return m * ld < kMax && (tok0 + tokens) * ld + rows < kMax;
 }
 
+// Whether the several-row head of a matrix runs as lmhead_tile_kernel rather
+// than the older several-row kernels.  Every workgroup of it first stages its
+// token rows (80 KB at 8 rows of 2560 columns), so matrices of fewer than two
+// 16-row tiles a CU, four at 5 to 8 rows, stay on the older ones
+// (lmhead_batch_kernel, 2560 x 4000: 12 against 13 us at 2 rows, 12 against 18
+// at 8; 2560 x 9000: 23 against 18 at 2, 23 against 25 at 8; 2560 x 24000 at 8:
+// 40 against 30; lmhead_stream_kernel, 16 rows, 2560 x 4000: 13 against 20, x
+// 8500: 25 against 26, x 12300: 31 against 28; 24 rows, x 4000: 20 against 21,
+// x 8500: 37 against 31).
+constexpr bool head_tiled(int64_t rows, int64_t m, int64_t cus) {
+    return (rows + 15) / 16 * ((m + 15) / 16) > (m > 4 && m <= 8 ? 4 : 2) * cus;
+}
+
+// Whether a linear of m >= 2 rows without a norm is faster with the one-row
+// kernel run per row (the same bits) than with the several-row kernels.  Those
+// read the weights once per 8 to 16 rows but stage the rows in LDS first
+// (2560 columns: 9 to 15 us before the first product), the one-row kernel
+// starts at once and reads them per row, from L2 where the matrix fits.
+// Estimates in us fitted to both sides at 4760 sizes (8 to 2560 columns, 16 to
+// 128256 rows, 2 to 64 tokens, bf16 and int8), one-row / several-row: bf16,
+// 2560 x 1000, 2 rows 7.1 / 10.8, 16 rows 9.0 / 11.5, 32 rows 13.4 / 12.1; 2560
+// x 4000, 2 rows 8.9 / 12.0, 4 rows 14.2 / 12.0; int8, 2560 x 1000, 16 rows 9.1
+// / 15.6; 2560 x 16000, 2 rows 15.9 / 19.6, 3 rows 22.0 / 19.5.
+constexpr bool head_row_by_row(int64_t rows, int64_t cols, int64_t m, bool q8, int64_t cus) {
+    const double mb = (double)rows * (double)cols * (q8 ? 1e-6 : 2e-6);  // the weights
+    const double one = (rows <= 32 ? 4.4 : 6.2) + (mb <= 5.5 ? 0.067 : 0.085) * mb * (double)m;
+    const bool big = m > 8;  // 16-token groups
+    const double reads = mb * (double)(big ? (m + 15) / 16 : 1);
+    const double several =
+        head_tiled(rows, m, cus)
+            ? 5.8 + 0.0012 * (double)cols + 0.146 * reads
+            : (big && q8 ? 5.3 : 4.1) + (!big ? 0.0017 : q8 ? 0.0023 : 0.0027) * (double)cols + 0.13 * reads;
+    return one <= several;
+}
+
 }  // namespace lbt

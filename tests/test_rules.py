@@ -15,6 +15,10 @@ extern "C" {
 int lean_offsets_fit(long m, long ld, long tok0, long tokens, long rows) {
     return lbt::lean_offsets_fit(m, ld, tok0, tokens, rows);
 }
+int head_tiled(long rows, long m, long cus) { return lbt::head_tiled(rows, m, cus); }
+int head_row_by_row(long rows, long cols, long m, int q8, long cus) {
+    return lbt::head_row_by_row(rows, cols, m, q8 != 0, cus);
+}
 }
 """
 
@@ -29,6 +33,8 @@ def rules(tmp_path_factory):
     assert r.returncode == 0, r.stderr
     lib = C.CDLL(str(so))
     lib.lean_offsets_fit.argtypes = [C.c_long] * 5
+    lib.head_tiled.argtypes = [C.c_long] * 3
+    lib.head_row_by_row.argtypes = [C.c_long] * 3 + [C.c_int, C.c_long]
     return lib
 
 
@@ -68,3 +74,17 @@ def test_no_launch_keeps_per_process_state():
     for src in sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp")):
         for n, line in enumerate(src.read_text().splitlines(), 1):
             assert not re.match(r"\s+static (?!const|inline|_)", line), f"{src.name}:{n}: {line.strip()}"
+
+
+# us on an MI355X, row by row and with the several-row kernels
+@pytest.mark.parametrize("q8,cols,rows,m,one,several", [
+    (0, 2560, 16, 64, 4.5, 9.9), (0, 2560, 64, 24, 6.0, 10.2), (0, 2560, 1000, 2, 7.1, 10.8), (0, 2560, 1000, 8, 7.2, 10.7),
+    (0, 2560, 1000, 48, 18.0, 12.8), (0, 2560, 2000, 4, 8.9, 11.2), (0, 2560, 4000, 2, 8.9, 12.0), (0, 2560, 4000, 5, 18.6, 12.1),
+    (0, 2560, 4000, 16, 46.7, 13.0), (0, 2560, 40000, 8, 230.3, 46.0), (0, 2048, 12000, 4, 31.6, 16.5), (0, 1280, 12000, 2, 12.1, 16.8),
+    (0, 1000, 16000, 3, 20.2, 14.2), (0, 512, 4000, 8, 9.4, 4.8), (0, 64, 40000, 64, 453.1, 40.6), (1, 64, 16, 9, 4.4, 5.9),
+    (1, 2560, 300, 16, 7.3, 15.2), (1, 2560, 1000, 16, 9.1, 15.6), (1, 2560, 1000, 64, 21.4, 16.4), (1, 2560, 4000, 2, 8.2, 11.3),
+    (1, 2560, 4000, 8, 16.0, 11.0), (1, 2560, 16000, 2, 15.9, 19.6), (1, 2560, 16000, 4, 27.8, 19.6), (1, 1000, 1000, 8, 7.8, 6.2),
+    (1, 1000, 300, 9, 7.2, 8.4), (1, 512, 40000, 24, 176.7, 23.5),
+])
+def test_several_row_linears_take_the_faster_kernel(rules, q8, cols, rows, m, one, several):
+    assert min(one, several) * 1.05 >= (one if rules.head_row_by_row(rows, cols, m, q8, 256) else several)
