@@ -345,12 +345,7 @@ int launch_attention_tile(lbt_ctx* ctx, const float* q, int m, int nh, int kvh, 
                           const uint16_t* kc, const uint16_t* vc, int cap, float scaling, float* o, float* ml) {
     const int ks = attn_split_keys(rp.vis_max);
     if (hd != kHd || m < 2 || rp.tok_pos || rp.pos_dev || ks > kTileLds) return 1;
-    // From five (row, KV head, split) tasks per CU on: below, 16-row tiles
-    // leave SIMDs idle and a wavefront's chain of 64 keys (12 us) is longer
-    // than the workgroup per task that serves those sizes (2B shape, 64
-    // tokens 12.5 against 7.8 us, 128 tokens 12.9 against 12.7, 200 tokens 13.2
-    // against 17.2; 50 tokens behind 700 13.5 against 17.7).
-    if (ctx->tune.attn_tile < 0 && (long)m * kvh * attn_splits(rp.vis_max) <= 5L * ctx->cus) return 1;
+    if (ctx->tune.attn_tile < 0 && !attn_tiles_pay(m, rp.pos0, nh, kvh, attn_splits(rp.vis_max), ks)) return 1;
     const int ntiles = (rp.pos0 + m - 1) / kTileRows - rp.pos0 / kTileRows + 1;
     const int scw = (ks + 63) / 64 * 64 * kTileRows;
     hipEvent_t e0, e1;

@@ -16,6 +16,29 @@ constexpr bool lean_offsets_fit(int64_t m, int64_t ld, int64_t tok0, int64_t tok
     return m * ld < kMax && (tok0 + tokens) * ld + rows < kMax;
 }
 
+// Whether the attention of m rows from position pos0 (head_dim 128) is faster
+// in 16-row tiles (attention_tile_kernel) than in the kernels of one workgroup
+// or wavefront per (row, KV head, split).  A tile wavefront runs its split's
+// keys one after another (12 us at 64 keys, 30 at 220), so there has to be
+// enough work to keep the other kernels busy for longer: theirs goes by the
+// (query head, visible key) pairs and by the workgroups, of which the more
+// heads share one the longer each lasts and the cheaper a pair is.  Fitted to
+// both sides at 1872 sizes (2 to 512 rows at positions 0 to 3500, 13 groupings
+// of 2 to 32 heads; the line is within 0.3 us of the faster side on the other
+// kernels' and 0.8 us on the tiles').  us workgroup / tile: 20 / 5 heads, 100
+// rows 10.5 / 12.6, 160 rows 14.9 / 13.1, 17 rows behind 3500 24.9 / 33; 8 / 8
+// heads, 160 rows 9.3 / 12.9, 17 rows behind 2000 13.3 / 18.9, 50 rows there
+// 35 / 21; 4 / 4 heads, 33 rows behind 700 7.4 / 12.1.
+constexpr bool attn_tiles_pay(int64_t m, int64_t pos0, int64_t nh, int64_t kvh, int64_t splits, int64_t split_keys) {
+    const int64_t gh = nh / kvh;  // heads per workgroup: 1, 2 or 4, other groups head by head
+    const double groups = (double)(m * splits * (gh == 1 || gh == 2 || gh == 4 ? kvh : nh));
+    const double pairs = (double)nh * ((double)m * (double)pos0 + 0.5 * (double)m * (double)(m + 1));
+    const double other = gh == 4   ? 5.2e-6 * pairs + 3.15e-3 * groups
+                         : gh == 2 ? 11.2e-6 * pairs + 1.42e-3 * groups
+                                   : 13.4e-6 * pairs + 0.86e-3 * groups;
+    return other > 1.9 + 0.059 * (double)split_keys;
+}
+
 // Whether the several-row head of a matrix runs as lmhead_tile_kernel rather
 // than the older several-row kernels.  Every workgroup of it first stages its
 // token rows (80 KB at 8 rows of 2560 columns), so matrices of fewer than two

@@ -19,6 +19,9 @@ int head_tiled(long rows, long m, long cus) { return lbt::head_tiled(rows, m, cu
 int head_row_by_row(long rows, long cols, long m, int q8, long cus) {
     return lbt::head_row_by_row(rows, cols, m, q8 != 0, cus);
 }
+int attn_tiles_pay(long m, long pos0, long nh, long kvh, long splits, long keys) {
+    return lbt::attn_tiles_pay(m, pos0, nh, kvh, splits, keys);
+}
 }
 """
 
@@ -35,6 +38,7 @@ def rules(tmp_path_factory):
     lib.lean_offsets_fit.argtypes = [C.c_long] * 5
     lib.head_tiled.argtypes = [C.c_long] * 3
     lib.head_row_by_row.argtypes = [C.c_long] * 3 + [C.c_int, C.c_long]
+    lib.attn_tiles_pay.argtypes = [C.c_long] * 6
     return lib
 
 
@@ -88,3 +92,20 @@ def test_no_launch_keeps_per_process_state():
 ])
 def test_several_row_linears_take_the_faster_kernel(rules, q8, cols, rows, m, one, several):
     assert min(one, several) * 1.05 >= (one if rules.head_row_by_row(rows, cols, m, q8, 256) else several)
+
+
+# us of the other kernels and of the 16-row tiles
+@pytest.mark.parametrize("heads,kv,pos0,m,other,tiles", [
+    (20, 5, 0, 64, 7.9, 13.1), (20, 5, 0, 100, 10.5, 13.0), (20, 5, 0, 160, 14.9, 13.1), (20, 5, 0, 512, 55.7, 35.8),
+    (20, 5, 700, 24, 14.4, 12.2), (20, 5, 2000, 17, 18.1, 19.6), (20, 5, 2000, 50, 34.3, 32.3), (20, 5, 3500, 17, 24.9, 33.2),
+    (20, 5, 3500, 64, 83.8, 48.2), (8, 8, 0, 100, 6.7, 12.9), (8, 8, 0, 160, 9.3, 13.2), (8, 8, 0, 200, 20.0, 13.1),
+    (8, 8, 700, 17, 7.4, 12.2), (8, 8, 700, 50, 16.7, 12.3), (8, 8, 2000, 17, 13.3, 19.1), (8, 8, 2000, 50, 35.4, 21.4),
+    (8, 8, 3500, 17, 24.4, 31.7), (4, 4, 0, 160, 6.5, 12.8), (4, 4, 700, 33, 7.6, 12.2), (4, 4, 2000, 100, 42.8, 22.9),
+    (32, 32, 0, 50, 7.0, 12.0), (32, 32, 0, 100, 20.6, 12.8), (8, 1, 2000, 17, 13.1, 19.1), (8, 1, 2000, 128, 90.0, 23.4),
+    (24, 12, 0, 50, 6.3, 12.3), (24, 12, 300, 64, 25.2, 13.4), (16, 2, 700, 9, 8.0, 12.0), (6, 2, 0, 200, 17.2, 13.0),
+])
+def test_prefill_attention_takes_the_faster_kernel(rules, heads, kv, pos0, m, other, tiles):
+    vis = pos0 + m
+    keys = max(64, -(-vis // 16))
+    pick = rules.attn_tiles_pay(m, pos0, heads, kv, -(-vis // keys), keys)
+    assert min(other, tiles) * 1.05 >= (tiles if pick else other)
