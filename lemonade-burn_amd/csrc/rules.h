@@ -74,4 +74,20 @@ constexpr bool head_row_by_row(int64_t rows, int64_t cols, int64_t m, bool q8, i
     return one <= several;
 }
 
+// Whether a prefill GEMM outside the one-workgroup-per-CU kernel takes 128 x
+// 128 tiles (t128 of them) rather than 64 x 64 (t64).  A round of 64 x 64 costs
+// 1.6 of their MFMA tiles (half the reuse of either operand), and 128 x 128
+// tiles that leave each CU at most one workgroup, one wavefront per SIMD, 4.6
+// instead of 4; 5.6 with an epilogue as long as that of q/k/v or of blocks
+// that straddle two matrices (2B shape, o and down at 850 tokens, 140 tiles:
+// 22.5 us against 26.6 on 560 of 64 x 64; at 768, 480 of them in two rounds:
+// 22.4 against 18.7; q/k/v at 768: 27.5 against 25.1, at 850: 27.8 against 29.6;
+// three matrices of 1000 rows, 700 tokens: 10.7 against 8.6 at 256 columns,
+// 13.3 against 12.1 at 1000, 1000 tokens and 4096 columns: 27.6 against 24.7).
+constexpr bool gemm_128_tiles(int64_t t128, int64_t t64, bool long_epilogue) {
+    const int64_t c64 = (t64 + 255) / 256 * 16;
+    const int64_t c128 = t128 > 256 ? (t128 + 255) / 256 * 40 : long_epilogue ? 56 : 46;
+    return c128 <= c64;
+}
+
 }  // namespace lbt

@@ -1301,16 +1301,13 @@ int launch_ternary_mfma(lbt_ctx* ctx, const TernaryOp& op_in) {
     // of 2 x 2 per SIMD, two workgroups per CU), 1 per 64 x 64 tile; ties go
     // to the one-workgroup-per-CU kernel
     const long c3 = (t3 + 255) / 256 * 8, c3n = (t3n + 255) / 256 * 6;
-    // 128 x 128 or 64 x 64 tiles: a round of 64 x 64 costs 1.6 (half the reuse
-    // of either operand), and 128 x 128 tiles that leave each CU at most one
-    // workgroup, one wavefront per SIMD, 4.6 instead of 4, 5.6 with the q/k/v
-    // epilogue (2B shape, o and down at 850 tokens, 140 tiles: 22.5 us against 26.6
-    // on 560 of 64 x 64; at 768, 480 of them in two rounds: 22.4 against 18.7;
-    // q/k/v at 768: 27.5 against 25.1, at 850: 27.8 against 29.6)
+    // 128 x 128 or 64 x 64 tiles (gemm_128_tiles); a matrix that does not end
+    // on a wavefront block's 64 rows leaves blocks in two matrices
     const long t64 = (long)g64.x * g64.y;
-    const long c64 = (t64 + 255) / 256 * 16;
-    const long c128 = t128 > 256 ? (t128 + 255) / 256 * 40 : op.out_mode == kOutQKV ? 56 : 46;
-    const bool use128 = c128 <= c64;
+    bool straddle = false;
+    if (op.out_mode != kOutRelu2)
+        for (int i = 0, end = 0; i + 1 < op.nmat; i++) straddle |= (end += op.rows[i]) % 64 != 0;
+    const bool use128 = gemm_128_tiles(t128, t64, straddle || op.out_mode == kOutQKV);
     const long c2 = use128 ? (t128 + 255) / 256 * 4 : (t64 + 255) / 256;
     int g3pick = c3n < c3 ? (t3n >= kG3MinTiles ? 2 : 0) : (t3 >= kG3MinTiles ? 1 : 0);
     if (g3pick != 0 && (g3pick == 2 ? c3n : c3) > c2) g3pick = 0;

@@ -22,6 +22,9 @@ int head_row_by_row(long rows, long cols, long m, int q8, long cus) {
 int attn_tiles_pay(long m, long pos0, long nh, long kvh, long splits, long keys) {
     return lbt::attn_tiles_pay(m, pos0, nh, kvh, splits, keys);
 }
+int gemm_128_tiles(long t128, long t64, int long_epilogue) {
+    return lbt::gemm_128_tiles(t128, t64, long_epilogue != 0);
+}
 }
 """
 
@@ -39,6 +42,7 @@ def rules(tmp_path_factory):
     lib.head_tiled.argtypes = [C.c_long] * 3
     lib.head_row_by_row.argtypes = [C.c_long] * 3 + [C.c_int, C.c_long]
     lib.attn_tiles_pay.argtypes = [C.c_long] * 6
+    lib.gemm_128_tiles.argtypes = [C.c_long, C.c_long, C.c_int]
     return lib
 
 
@@ -109,3 +113,14 @@ def test_prefill_attention_takes_the_faster_kernel(rules, heads, kv, pos0, m, ot
     keys = max(64, -(-vis // 16))
     pick = rules.attn_tiles_pay(m, pos0, heads, kv, -(-vis // keys), keys)
     assert min(other, tiles) * 1.05 >= (tiles if pick else other)
+
+
+# us with 64 x 64 and 128 x 128 tiles
+@pytest.mark.parametrize("rows,m,small,large", [
+    ((1503, 203), 1250, 12.2, 13.6), ((1000, 1000, 1000), 700, 8.6, 10.6), ((1000, 1000, 1000), 1000, 24.7, 27.6),
+    ((2560,), 850, 26.6, 22.5), ((2560,), 768, 18.7, 22.4)])
+def test_prefill_gemms_take_the_faster_tile(rules, rows, m, small, large):
+    total, ends = sum(rows), [sum(rows[:i + 1]) for i in range(len(rows) - 1)]
+    t128, t64 = -(-total // 128) * -(-m // 128), -(-total // 64) * -(-m // 64)
+    pick = rules.gemm_128_tiles(t128, t64, int(any(e % 64 for e in ends)))
+    assert pick == (large < small)
