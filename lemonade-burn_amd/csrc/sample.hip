@@ -31,6 +31,8 @@
 #include "lbt_device.h"
 #include "lbt_internal.h"
 
+#include <type_traits>
+
 namespace lbt {
 
 namespace {
@@ -69,10 +71,11 @@ struct SampleShared {
 
 // Per-chunk results of the candidate pass: the largest total-order key of
 // the chunk (sample_max_kernel), then its candidates' weight sum, the
-// smallest key of a NaN p and the largest key (sample_cand_kernel).
+// smallest key of a NaN p, the largest key and the row's largest total-order
+// key (sample_cand_kernel).
 struct ChunkSum {
     unsigned long long w, nan_s, smax;
-    unsigned cmax, pad;
+    unsigned cmax, rmax;
 };
 
 // Ascending key of the IEEE total order (total_cmp) of x's bits.
@@ -90,6 +93,24 @@ __device__ __forceinline__ unsigned long long sample_key(float x, unsigned i, in
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
+}
+// Inclusive sums over the lanes (DPP: a step is two moves and an add, where
+// __shfl_up waits for the LDS pipe).  All lanes call.
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long v) {
+    auto step = [&](auto c, auto r) {
+        constexpr int ctrl = decltype(c)::value, rows = decltype(r)::value;
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, ctrl, rows, 0xf, false);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(v >> 32), ctrl, rows, 0xf, false);
+        v += (unsigned long long)hi << 32 | lo;
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1, 2, 4, 8
+    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15 into rows 1, 3
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31 into rows 2, 3
     return v;
 }
 __device__ __forceinline__ unsigned long long wave_min(unsigned long long v) {
@@ -371,6 +392,18 @@ __global__ __launch_bounds__(kCT) void sample_cand_kernel(SampleArgs a) {
     int ib = 1;
     while (ib < 32 && (1u << ib) < (unsigned)V) ib++;
     const int c0 = g * kChunk, c1 = c0 + kChunk < V ? c0 + kChunk : V;
+    // the coarse histogram of a list that may need sample_cut: a thread adds
+    // its runs of one bin, since atomics on one address follow one another
+    // (a row of 5000 equal logits: 67 us a call, 70 with an atomic per logit)
+    const bool coarse = V > kLdsCand;
+    int rbin = 0;
+    unsigned long long rw = 0;
+    unsigned rn = 0;
+    auto flush = [&] {
+        if (!rn) return;
+        atomicAdd(&xh[rbin], rw);
+        atomicAdd(&xc[rbin], rn);
+    };
     unsigned long long wsum = 0, nan_s = kNone, smax = 0;
     for (int i0 = c0; i0 < c1; i0 += kCT) {
         const int i = i0 + tid;
@@ -388,9 +421,16 @@ __global__ __launch_bounds__(kCT) void sample_cand_kernel(SampleArgs a) {
                 w = (unsigned long long)(p * 0x1p45f);
                 keep = w != 0;
                 wsum += w;
-                if (keep) {
-                    atomicAdd(&xh[x_bin(x)], w);
-                    atomicAdd(&xc[x_bin(x)], 1u);
+                if (coarse && keep) {
+                    const int bin = x_bin(x);
+                    if (bin != rbin) {
+                        flush();
+                        rbin = bin;
+                        rw = 0;
+                        rn = 0;
+                    }
+                    rw += w;
+                    rn++;
                 }
             }
         }
@@ -402,6 +442,7 @@ __global__ __launch_bounds__(kCT) void sample_cand_kernel(SampleArgs a) {
             if (keep) lc[base + (unsigned)__popcll(m & ((1ull << lane) - 1))] = Cand{s, w};
         }
     }
+    flush();
     wsum = wave_sum(wsum);
     nan_s = wave_min(nan_s);
     smax = wave_max(smax);
@@ -421,6 +462,7 @@ __global__ __launch_bounds__(kCT) void sample_cand_kernel(SampleArgs a) {
         sums[g].w = W;
         sums[g].nan_s = ns;
         sums[g].smax = sm;
+        sums[g].rmax = mk;
         base = cnt ? atomicAdd(&a.ncand[row], cnt) : 0u;
     }
     __syncthreads();
@@ -447,12 +489,14 @@ __device__ __forceinline__ unsigned long long draw_target(unsigned long long u, 
 // read once against a threshold below that bin, the few that pass are
 // computed again (the same key and weight) and those of the bins kept written
 // over the row's list.  Returns their number, 0 to go on with the whole list.
-// Six rounds over a 2 MB list by one workgroup took 290 us a call (4 rows of
-// 128256 normal logits of deviation 2.5, temperature 0.8, top-p 0.95: 308 us
-// in all), with the cut 95 in all; top-k 40 330 -> 64, no cut 238 -> 72.  A row
-// of which more than half stays pays 3 us for the look.
-__device__ unsigned sample_cut(const SampleArgs& a, int row, const float* lg, int V, int ib, unsigned n,
-                               unsigned long long Wall, unsigned long long u, float mx, Cand* gc, SampleShared& sh) {
+// Six rounds over a 2 MB list by one workgroup bounded the call: 4 rows of
+// 128256 normal logits of deviation 2.5 and 24 larger ones, temperature 0.8 and
+// top-p 0.95, 281 us a call of ten in a row, with the cut 69; top-k 40 331 ->
+// 63, no limit 241 -> 117.  A row of which more than half stays pays 1.7 us for
+// the histogram and the look (4 rows of 5000 logits of deviation 1: 49.6 ->
+// 51.3; 3 us with a scan through the LDS pipe and the histogram read here).
+__device__ unsigned sample_cut(const SampleArgs& a, const float* lg, int V, int ib, unsigned n, unsigned long long Wall,
+                               unsigned long long u, float mx, Cand* gc, SampleShared& sh) {
     const int tid = threadIdx.x, lane = tid & 63;
     const unsigned long long kk = (a.top_k > 0 && a.top_k < (unsigned long long)V) ? a.top_k : (unsigned long long)V;
     const bool by_count = kk < n;
@@ -463,36 +507,31 @@ __device__ unsigned sample_cut(const SampleArgs& a, int row, const float* lg, in
         unsigned long long h[PL], sum = 0;
 #pragma unroll
         for (int j = 0; j < PL; j++) {
-            const size_t b = (size_t)row * kXB + PL * lane + j;
-            h[j] = by_count ? (unsigned long long)gload(a.xcnt + b) : gload(a.xhist + b);
+            h[j] = by_count ? (unsigned long long)sh.bcnt[PL * lane + j] : sh.hist[PL * lane + j];
             sum += h[j];
         }
-        unsigned long long inc = sum;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned long long v = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += v;
-        }
-        unsigned long long run = inc - sum;
+        unsigned long long run = wave_scan(sum) - sum;
         unsigned found = kXB - 1;
 #pragma unroll
         for (int j = 0; j < PL; j++) {
             run += h[j];
             if (found == kXB - 1 && run >= target) found = PL * lane + j;
         }
-        const unsigned long long first = wave_min((unsigned long long)found);
+        const unsigned long long hit = __ballot(found != kXB - 1);
+        const unsigned first = hit ? __builtin_amdgcn_readlane(found, __ffsll(hit) - 1) : kXB - 1;
         // candidates up to that bin, and in the next two, which may pass the threshold below
-        unsigned long long upto = 0, near = 0;
+        unsigned upto = 0, near = 0;
 #pragma unroll
         for (int j = 0; j < PL; j++) {
-            const unsigned b = PL * lane + j, cb = gload(a.xcnt + (size_t)row * kXB + b);
+            const unsigned b = PL * lane + j, cb = sh.bcnt[b];
             if (b <= first) upto += cb;
             if (b <= first + 2) near += cb;
         }
-        upto = wave_sum(upto);
-        near = wave_sum(near);
-        if (lane == 0) {
-            sh.sel_bin = (unsigned)first;
+        const unsigned long long both = wave_scan((unsigned long long)near << 32 | upto);
+        upto = (unsigned)both;
+        near = (unsigned)(both >> 32);
+        if (lane == 63) {
+            sh.sel_bin = first;
             sh.cnt = 0;
             sh.sel_cnt = 0;
             sh.sel_below = upto > n / 2 || near > (unsigned)kIdx;  // a row too flat to cut
@@ -661,6 +700,12 @@ __global__ __launch_bounds__(kST) void sample_kernel(SampleArgs a) {
     const int G = a.G;
     const ChunkSum* sums = a.sums + (size_t)row * G;
     unsigned long long wsum = 0, nan_s = kNone, smax = 0;
+    const unsigned mk = gload(&sums[0].rmax);
+    if (V > kLdsCand)  // the row's coarse histogram, for sample_cut
+        for (int b = tid; b < kXB; b += kST) {
+            sh.hist[b] = gload(a.xhist + (size_t)row * kXB + b);
+            sh.bcnt[b] = gload(a.xcnt + (size_t)row * kXB + b);
+        }
     for (int g = tid; g < G; g += kST) {
         wsum += gload(&sums[g].w);
         const unsigned long long ns = gload(&sums[g].nan_s), sm = gload(&sums[g].smax);
@@ -680,14 +725,8 @@ __global__ __launch_bounds__(kST) void sample_kernel(SampleArgs a) {
     const unsigned long long u = st >> 40;
     unsigned nl = n;  // elements of the list
     if (n > (unsigned)kLdsCand && nan_s == kNone) {
-        unsigned long long cm = 0;
-        for (int g = tid; g < G; g += kST) {
-            const unsigned long long k = gload(&sums[g].cmax);
-            cm = k > cm ? k : cm;
-        }
-        const unsigned mk = (unsigned)block_red<2>(cm, sh.red2);
         const float mx = __uint_as_float((mk & 0x80000000u) ? (mk & 0x7fffffffu) : ~mk);
-        const unsigned c = sample_cut(a, row, lg, V, ib, n, Wall, u, mx, gc, sh);
+        const unsigned c = sample_cut(a, lg, V, ib, n, Wall, u, mx, gc, sh);
         if (c) nl = c;
     }
     // few candidates: copied into LDS
