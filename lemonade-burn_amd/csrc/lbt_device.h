@@ -157,6 +157,18 @@ __device__ __forceinline__ float lbt_expf(float x) {
     return p * __uint_as_float((uint32_t)(ni + 127) << 23);
 }
 
+// v[l ^ M] by DPP, M = 1, 2, 4 or 8.  Every lane of the wavefront must be active.
+template <int M>
+__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "xor distance");
+    const int iv = (int)v;
+    if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xf, 0xf, false);
+    if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xf, 0xf, false);
+    if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x128, 0xf, 0xf, false);
+    const int p = __builtin_amdgcn_update_dpp(0, iv, 0x12C, 0xf, 0x5, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(p, iv, 0x124, 0xf, 0xA, false);
+}
+
 // Cross-lane exchange without LDS: xor_pair<M>(v) returns (a, b) with
 // {a, b} = {v[l], v[l ^ M]} at every lane l (the order within the pair may
 // differ between lanes, which commutative combines do not see).
@@ -177,17 +189,8 @@ __device__ __forceinline__ void xor_pair(uint32_t v, uint32_t& a, uint32_t& b) {
         a = r[0];
         b = r[1];
     } else {
-        const int iv = (int)v;
-        int p;
-        if constexpr (M == 1) p = __builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xf, 0xf, false);
-        else if constexpr (M == 2) p = __builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xf, 0xf, false);
-        else if constexpr (M == 8) p = __builtin_amdgcn_update_dpp(0, iv, 0x128, 0xf, 0xf, false);
-        else {
-            p = __builtin_amdgcn_update_dpp(0, iv, 0x12C, 0xf, 0x5, false);
-            p = __builtin_amdgcn_update_dpp(p, iv, 0x124, 0xf, 0xA, false);
-        }
         a = v;
-        b = (uint32_t)p;
+        b = xor_lane<M>(v);
     }
 }
 

@@ -358,9 +358,8 @@ __device__ __forceinline__ void epi32_relu2(const GemvArgs& a, v16i (&acc)[MS][N
             for (int s = 0; s < NS; s++) {
                 const int keep = odd ? acc[ms][s][r + 1] : acc[ms][s][r];
                 const int send = odd ? acc[ms][s][r] : acc[ms][s][r + 1];
-                uint32_t own, got;
-                xor_pair<1>((uint32_t)send, own, got);
-                const int dg = (odd ? (int)got : keep) - qs, du = (odd ? keep : (int)got) - qs;
+                const int got = (int)xor_lane<1>((uint32_t)send);
+                const int dg = (odd ? got : keep) - qs, du = (odd ? keep : got) - qs;
                 const float y0 = (float)dg * ig;
                 const float u = (float)du * iu;
                 const float rl = y0 > 0.0f ? y0 : 0.0f;
