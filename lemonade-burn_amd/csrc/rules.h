@@ -61,7 +61,8 @@ constexpr bool head_tiled(int64_t rows, int64_t m, int64_t cus) {
 // 128256 rows, 2 to 64 tokens, bf16 and int8), one-row / several-row: bf16,
 // 2560 x 1000, 2 rows 7.1 / 10.8, 16 rows 9.0 / 11.5, 32 rows 13.4 / 12.1; 2560
 // x 4000, 2 rows 8.9 / 12.0, 4 rows 14.2 / 12.0; int8, 2560 x 1000, 16 rows 9.1
-// / 15.6; 2560 x 16000, 2 rows 15.9 / 19.6, 3 rows 22.0 / 19.5.
+// / 15.6; 2560 x 16000, 2 rows 15.9 / 19.6, 3 rows 22.0 / 19.5.  The one-row
+// kernel has the rows in its grid's y, which ends at 65535.
 constexpr bool head_row_by_row(int64_t rows, int64_t cols, int64_t m, bool q8, int64_t cus) {
     const double mb = (double)rows * (double)cols * (q8 ? 1e-6 : 2e-6);  // the weights
     const double one = (rows <= 32 ? 4.4 : 6.2) + (mb <= 5.5 ? 0.067 : 0.085) * mb * (double)m;
@@ -71,7 +72,7 @@ constexpr bool head_row_by_row(int64_t rows, int64_t cols, int64_t m, bool q8, i
         head_tiled(rows, m, cus)
             ? 5.8 + 0.0012 * (double)cols + 0.146 * reads
             : (big && q8 ? 5.3 : 4.1) + (!big ? 0.0017 : q8 ? 0.0023 : 0.0027) * (double)cols + 0.13 * reads;
-    return one <= several;
+    return m <= 65535 && one <= several;
 }
 
 // Whether a prefill GEMM outside the one-workgroup-per-CU kernel takes 128 x

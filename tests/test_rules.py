@@ -98,6 +98,13 @@ def test_several_row_linears_take_the_faster_kernel(rules, q8, cols, rows, m, on
     assert min(one, several) * 1.05 >= (one if rules.head_row_by_row(rows, cols, m, q8, 256) else several)
 
 
+def test_more_rows_than_a_grid_holds_stay_on_the_several_row_kernels(rules):
+    for rows in (1, 16, 32, 33, 1000):
+        for cols in (8, 64, 2560):
+            assert not any(rules.head_row_by_row(rows, cols, m, q8, 256) for m in (65536, 70000, 1 << 30)
+                           for q8 in (0, 1))
+
+
 # us of the other kernels and of the 16-row tiles
 @pytest.mark.parametrize("heads,kv,pos0,m,other,tiles", [
     (20, 5, 0, 64, 7.9, 13.1), (20, 5, 0, 100, 10.5, 13.0), (20, 5, 0, 160, 14.9, 13.1), (20, 5, 0, 512, 55.7, 35.8),
