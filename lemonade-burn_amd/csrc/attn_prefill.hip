@@ -1,5 +1,6 @@
 // attn_prefill.hip -- attention splits of a prefill's rows on the f32 matrix
-// cores, with the partials of attention_split_ku (attn_common.h) bit for bit.
+// cores, with the partials of attention_split_ku (attn_common.h) bit for bit
+// but for the sign of a zero (below).
 //
 // Reference: crates/lb-model/src/model.rs:349-357 (GQA attention of a prompt).
 //
@@ -98,8 +99,11 @@ __device__ __forceinline__ float exp_le0(float x) {
 // of its key, so the four dims of a lane are 8 contiguous bytes of V and 16
 // of the output.
 //
-// A key that a row does not see has p = 0 there (fma(0, v, acc) = acc, acc
-// never -0).  That needs v finite: a non-finite V value among the tile's
+// A key that a row does not see has p = 0 there: fma(0, v, acc) = acc, but for
+// an acc of -0 (every product so far below the denormals), which may become
+// +0.  A partial can so differ from attention_split_ku's in the sign of a
+// zero; the o projection's input is rounded to integers, which have none.
+// That needs v finite: a non-finite V value among the tile's
 // partly masked keys makes the wavefront redo PV row by row, each with the
 // keys past its own read as zeros.
 //

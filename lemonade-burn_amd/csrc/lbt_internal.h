@@ -187,7 +187,7 @@ int launch_quantize(lbt_ctx* ctx, const float* x, const float* norm_w, float eps
 int launch_bf16_linear(lbt_ctx* ctx, const uint16_t* w, int rows, int cols, const float* x, int m,
                        const float* norm_w, float eps, float* logits, unsigned long long* key, float* xn = nullptr);
 // Either head (rscale: int8 weights) for m already normalized rows on the f32
-// matrix cores, 4, 8 or 16 rows at a time, the one-token head's bits (head_tile.hip);
+// matrix cores, 4, 8, 12 or 16 rows at a time, the one-token head's bits (head_tile.hip);
 // returns 1 (nothing launched) for what it does not take.
 int launch_head_tile(lbt_ctx* ctx, const void* w, const float* rscale, int rows, int cols, const float* xn, int m,
                      float* logits, unsigned long long* key);

@@ -1,7 +1,9 @@
 """Several-row bf16 and int8 heads on the f32 matrix cores: every row's sums
 equal the one-row head's bit for bit, over ragged rows, columns past a chain's
-last chunk, token groups, unaligned inputs and sums whose products underflow."""
+last chunk, token groups, unaligned inputs and sums whose products underflow;
+and the greedy tokens they pick are the first largest logit's."""
 import ctypes as C
+import json
 
 import numpy as np
 import pytest
@@ -34,7 +36,8 @@ def linear_dev(ctx, fn, h, x, rows, offset=0):
 
 # rows: whole and ragged 16-row tiles, few and many a CU, an odd and an even
 # number a workgroup; cols: one to five chunks a chain, whole and cut; first
-# matrices that stay on the older kernels
+# matrices that stay on the older kernels, or (2560 x 4000 at 2 rows, 1001 x 648
+# at 2 to 50 of int8) go row by row
 @pytest.mark.parametrize("rows,cols", [(300, 8), (1001, 648), (4000, 2560), (16401, 8), (16409, 128),
                                        (17345, 512), (16399, 520), (18000, 1000),
                                        (16500, 1536), (16807, 2040), (16392, 2552), (16400, 2560), (24577, 2560)])
@@ -59,3 +62,52 @@ def test_several_rows_equal_one_row(ctx, rows, cols, q8):
     if q8:
         h.free()
     b.free()
+
+
+# Greedy tokens (the argmax keys of the several-row kernels): vocabularies above
+# their line, whole and ragged 16-row tiles; every token group (4, 8, 12 and 16
+# rows, one and two of them); every embedding row twice, so that each largest
+# logit is a tie of two rows that different workgroups hold.
+@pytest.mark.parametrize("vocab", [34000, 34009])
+def test_greedy_tokens_are_the_first_largest_logit(ctx, tmp_path, vocab):
+    import torch
+    from safetensors.torch import save_file
+
+    H, I, half = 640, 256, vocab // 2
+    rng = np.random.default_rng(vocab)
+    t = {}
+    names = ["self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj", "mlp.gate_proj",
+             "mlp.up_proj", "mlp.down_proj"]
+    for n, (r, c) in zip(names, [(H, H), (128, H), (128, H), (H, H), (I, H), (I, H), (H, I)]):
+        w = rng.integers(-1, 2, (r, c)).astype(np.int8)
+        t[f"model.layers.0.{n}.qweight"] = torch.from_numpy(np.ascontiguousarray(orc.pack(w)))
+        t[f"model.layers.0.{n}.wscale"] = torch.from_numpy(np.array([20.0], np.float32))
+    for n, k in (("input_layernorm", H), ("post_attention_layernorm", H), ("self_attn.attn_sub_norm", H),
+                 ("mlp.ffn_sub_norm", I)):
+        t[f"model.layers.0.{n}.weight"] = torch.ones(k)
+    t["model.norm.weight"] = torch.ones(H)
+    emb = rng.uniform(-1, 1, (vocab, H)).astype(np.float32)
+    emb[half:2 * half] = emb[:half]
+    t["model.embed_tokens.weight"] = torch.from_numpy(emb).to(torch.bfloat16)
+    save_file(t, str(tmp_path / "model.lbt.safetensors"), metadata={"format": "lemonade-burn-ternary", "version": "1"})
+    (tmp_path / "config.json").write_text(json.dumps({
+        "hidden_size": H, "intermediate_size": I, "num_attention_heads": 5, "num_key_value_heads": 1,
+        "num_hidden_layers": 1, "vocab_size": vocab, "rms_norm_eps": 1e-5, "rope_theta": 1e4,
+        "max_position_embeddings": 64, "hidden_act": "relu2", "tie_word_embeddings": True, "bos_token_id": 1}))
+    m = lbt_hip.Model.load(ctx, tmp_path)
+    for kind in (0, 1):
+        m.set_head(kind)
+        for nseq in (2, 6, 11, 16, 20, 30):
+            announce(f"greedy tokens of the several-row head, vocab={vocab} kind={kind} nseq={nseq}")
+            toks = rng.integers(0, vocab, nseq).astype(np.uint32)
+            for want in (True, False):
+                b = m.new_batch(nseq, 64)
+                b.fill_synthetic(9, 4)
+                logits, nxt = b.forward(toks, want)
+                b.free()
+                if want:
+                    first = logits.argmax(1)
+                    assert (first < half).any()
+                    assert (np.ptp(np.sort(logits, 1)[:, -2:], axis=1) == 0)[first < half].all()
+                assert np.array_equal(nxt, first)
+    m.free()

@@ -367,9 +367,9 @@ def test_memcpy_d2d_sizes(ctx):
 
 
 def test_batched_bf16_head_kernels_agree(ctx, ctx_with):
-    """The batched bf16 head on the weight-streaming kernel (default) and on
-    lmhead_batch_kernel (LBT_HEAD_BATCH_CLASSIC) give the same logits bit for
-    bit, at the 2B head's width for 16..64 rows."""
+    """The batched bf16 head on the matrix-core kernel (what 20000 rows take)
+    and on lmhead_batch_kernel (LBT_HEAD_BATCH_CLASSIC) give the same logits
+    bit for bit, at the 2B head's width for 16..64 rows."""
     rng = np.random.default_rng(31)
     rows, cols = 20000, 2560
     wb = orc.f32_to_bf16((rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)).reshape(rows, cols)
