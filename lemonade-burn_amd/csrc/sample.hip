@@ -784,9 +784,12 @@ int launch_sample(lbt_ctx* ctx, const float* logits, long ld, int rows, int voca
     a.xhist = (unsigned long long*)((char*)scratch + cand_bytes(rows, vocab) + sums_bytes(rows, vocab));
     a.xcnt = (unsigned*)((char*)a.xhist + xhist_bytes(rows));
     a.ncand = a.xcnt + (size_t)rows * kXB;
-    // the candidate pass over chunks of the row, then one workgroup per row
-    hipLaunchKernelGGL(sample_max_kernel, dim3(a.G, rows), dim3(kCT), 0, ctx->stream, a);
-    hipLaunchKernelGGL(sample_cand_kernel, dim3(a.G, rows), dim3(kCT), 0, ctx->stream, a);
+    // the candidate pass over chunks of the row (nothing to do where every row
+    // is an argmax), then one workgroup per row
+    if (rowp || !(p.temperature <= 0.0f)) {
+        hipLaunchKernelGGL(sample_max_kernel, dim3(a.G, rows), dim3(kCT), 0, ctx->stream, a);
+        hipLaunchKernelGGL(sample_cand_kernel, dim3(a.G, rows), dim3(kCT), 0, ctx->stream, a);
+    }
     hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(kST), 0, ctx->stream, a);
     LBT_HIP(ctx, hipGetLastError());
     return LBT_OK;
