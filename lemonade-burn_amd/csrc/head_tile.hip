@@ -48,7 +48,10 @@ constexpr int kMaxNch = 5;  // chunks per chain: columns up to 2560 (16 rows of 
 // chains), with the token rows in LDS and a whole tile a wavefront (16 rows of
 // bf16 160 us, with 64-byte pieces of a row a load 200), and with the chains
 // split over eight wavefronts, token rows in registers and an exchange of the
-// sums through LDS (150; 64 rows 477).
+// sums through LDS (150; 64 rows 477).  FULL (columns a multiple of 512, no
+// bounds test on a load) is worth 1 to 3%, at 16 rows of 512 columns 9%, and up to 28%
+// at 12 rows, where the test's registers add to what spills (128256 x 2560 bf16:
+// 128 against 155 us).
 template <int NCH, bool FULL, bool Q8, int TG, int RG, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void lmhead_tile_kernel(
     const void* W, const float* rscale, int rows, int cols, const float* xn, int m, int part_tiles, float* logits,
@@ -90,11 +93,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void lm
     // token rows; columns past the end are -0: a product of it with a zero
     // weight leaves every sum as it is
     auto swz = [](int t) { return (t & 1) + 4 * (t & 2); };
-    if (cols == 4 * G && ((uintptr_t)xn & 15) == 0) {
+    // every row starts aligned if the first does (cols is a multiple of 8); 2432
+    // columns, 8500 rows, 16 tokens: 32 us, value by value 50
+    if (((uintptr_t)xn & 15) == 0) {
         for (int i = tid; i < 4 * TG * G; i += NT) {
             const int t = i / G, g = i % G;
-            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (t < nt) v = gload((const f32x4*)(xn + (size_t)t * cols) + g);
+            f32x4 v = {-0.0f, -0.0f, -0.0f, -0.0f};
+            if (t < nt && (FULL || 4 * g < cols)) v = gload((const f32x4*)(xn + (size_t)t * cols) + g);
             *(f32x4*)(xs + 4 * (t * G + (g ^ swz(t)))) = v;
         }
     } else {
