@@ -71,7 +71,7 @@ constexpr bool head_row_by_row(int64_t rows, int64_t cols, int64_t m, bool q8, i
     const double several =
         head_tiled(rows, m, cus)
             ? 5.8 + 0.0012 * (double)cols + 0.146 * reads
-            : (big && q8 ? 5.3 : 4.1) + (!big ? 0.0017 : q8 ? 0.0023 : 0.0027) * (double)cols + 0.13 * reads;
+            : (big && q8 ? 5.3 : 4.1) + (!big ? 0.00175 : q8 ? 0.00235 : 0.00275) * (double)cols + 0.13 * reads;
     return m <= 65535 && one <= several;
 }
 

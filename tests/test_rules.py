@@ -87,7 +87,8 @@ def test_no_launch_keeps_per_process_state():
 # us on an MI355X, row by row and with the several-row kernels
 @pytest.mark.parametrize("q8,cols,rows,m,one,several", [
     (0, 2560, 16, 64, 4.5, 9.9), (0, 2560, 64, 24, 6.0, 10.2), (0, 2560, 1000, 2, 7.1, 10.8), (0, 2560, 1000, 8, 7.2, 10.7),
-    (0, 2560, 1000, 48, 18.0, 12.8), (0, 2560, 2000, 4, 8.9, 11.2), (0, 2560, 4000, 2, 8.9, 12.0), (0, 2560, 4000, 5, 18.6, 12.1),
+    (0, 2560, 1000, 16, 9.0, 11.5),
+    (0, 2560, 1000, 48, 18.0, 12.8), (0, 2560, 1500, 5, 8.7, 11.3), (0, 2560, 2000, 4, 8.9, 11.2), (0, 2560, 4000, 2, 8.9, 12.0), (0, 2560, 4000, 5, 18.6, 12.1),
     (0, 2560, 4000, 16, 46.7, 13.0), (0, 2560, 40000, 8, 230.3, 46.0), (0, 2048, 12000, 4, 31.6, 16.5), (0, 1280, 12000, 2, 12.1, 16.8),
     (0, 1000, 16000, 3, 20.2, 14.2), (0, 512, 4000, 8, 9.4, 4.8), (0, 64, 40000, 64, 453.1, 40.6), (1, 64, 16, 9, 4.4, 5.9),
     (1, 2560, 300, 16, 7.3, 15.2), (1, 2560, 1000, 16, 9.1, 15.6), (1, 2560, 1000, 64, 21.4, 16.4), (1, 2560, 4000, 2, 8.2, 11.3),
